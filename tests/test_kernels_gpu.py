@@ -87,6 +87,56 @@ def test_gemm_bf16_deep_k_ragged_m(gpu, M, N, K, n_acc):
     assert _rel(ss, (xf * xf).sum(-1)) < 1e-5
 
 
+@pytest.mark.parametrize("M,N,K,n_acc", [
+    (129, 2048, 1088, 1), (700, 2752, 2048, 2), (3001, 4096, 136, 1), (257, 2056, 1160, 1), (1500, 1024, 5640, 1),
+    (2000, 5632, 200, 2), (6000, 2048, 1000, 1), (4096, 4096, 128, 2)])
+def test_gemm_bf16_large_tiles(gpu, M, N, K, n_acc):
+    """256-column tiles of 128, 192 and 256 rows: row remainders, K steps that are odd in number or partial
+    (K % 64 != 0), residual and SwiGLU epilogues with the row scale, an output window; and an infinity in the
+    columns a partial step reads again."""
+    from torch_helion.hip import abi, ops
+
+    announce(f"gemm bf16 large tiles M={M} N={N} K={K} n_acc={n_acc}")
+    g = torch.Generator().manual_seed(M + N + K)
+    a = torch.randn(M, K, generator=g).bfloat16()
+    ws = [(torch.randn(K, N, generator=g) * 0.05).bfloat16() for _ in range(n_acc)]
+    ss = a.double().square().sum(-1)
+    r = torch.rsqrt(ss / K + 1e-5)[:, None]
+    acc = [a.to(gpu).double() @ w.to(gpu).double() for w in ws]
+    r = r.to(gpu)
+    o32 = torch.empty(M, N, device=gpu)
+    o16 = torch.empty(M, N, dtype=torch.bfloat16, device=gpu)
+    win = torch.full((M, 64), 7.0, device=gpu)
+    ssq = torch.empty(M, device=gpu)
+    kw = dict(sumsq=True, rscale_mask=(1 << n_acc) - 1, inv_k=1.0 / K, eps=1e-5, sumsq_out=ssq)
+    ad, packed = a.to(gpu), ops.pack_rhs([w.to(gpu) for w in ws], torch.bfloat16)
+    if n_acc == 1:
+        res = torch.randn(M, N, generator=g).to(gpu)
+        outs = [ops.EpiSpec(abi.EPI_ADD, o16, e=0), ops.EpiSpec(abi.EPI_ADD, o32, e=0),
+                ops.EpiSpec(abi.EPI_ACC, win, cols=(N - 64, N))]
+        ref, kw["extras"] = acc[0] * r + res.double(), [res]
+    else:
+        outs = [ops.EpiSpec(abi.EPI_SWIGLU, o16, a=0, b=1), ops.EpiSpec(abi.EPI_SWIGLU, o32, a=0, b=1),
+                ops.EpiSpec(abi.EPI_ACC, win, a=1, cols=(N - 64, N))]
+        ref = torch.nn.functional.silu(acc[0] * r) * (acc[1] * r)
+    ops.gemm(ops.GemmCall(M, N, K, n_acc, ad, packed, outs, **kw))
+    torch.cuda.synchronize()
+    # fp32 accumulation of exact bf16 products: K roundings of 2^-24 of the sum of magnitudes at most,
+    # far under 1e-5 of the largest output; SwiGLU's sigmoid uses the 1-ulp hardware exp and reciprocal
+    assert _rel(o32, ref) < 1e-5
+    assert torch.equal(o16, o32.bfloat16())
+    assert _rel(win, (acc[-1] * r)[:, N - 64:]) < 1e-5
+    assert _rel(ssq, ss) < 1e-5
+    if n_acc == 1:
+        # row 0 holds an infinity in a column that a partial last step reads twice: it counts once, in its row only
+        ad[0, K - 70] = float("inf")
+        ops.gemm(ops.GemmCall(M, N, K, 1, ad, packed, [ops.EpiSpec(abi.EPI_ACC, o32)]))
+        torch.cuda.synchronize()
+        w_row = ws[0][K - 70].to(gpu).float()
+        assert bool((o32[0] == torch.where(w_row == 0, torch.nan, torch.inf * w_row))[w_row != 0].all())
+        assert _rel(o32[1:], acc[0][1:]) < 1e-5
+
+
 @pytest.mark.parametrize("M,N,K,n_acc,mask", [(2000, 2192, 512, 1, 1), (2048, 2192, 512, 1, 0), (1000, 5000, 256, 1, 1),
                                               (2040, 1100, 512, 2, 2), (2048, 1100, 512, 1, 1), (2000, 700, 512, 1, 1)])
 def test_gemm_direct_two_blocks_per_cu(gpu, M, N, K, n_acc, mask):

@@ -40,66 +40,8 @@
 
 namespace th {
 
-// Block id -> output tile. Consecutive workgroups are dealt round-robin to the
-// 8 XCDs; remap so each XCD owns a contiguous range of logical tiles, then walk
-// that range in groups of 8 tile-rows so neighbouring blocks on one XCD share
-// lhs rows and rhs columns in that XCD's L2.
-__device__ __forceinline__ void map_tile_id(int pid, int tiles_m, int tiles_n, int& tm, int& tn) {
-  const int nb = tiles_m * tiles_n;
-  if ((nb & 7) == 0) pid = (pid & 7) * (nb >> 3) + (pid >> 3);
-  const int G = 8;
-  const int group = pid / (G * tiles_n);
-  const int first = group * G;
-  const int gm = min(tiles_m - first, G);
-  const int in_group = pid - group * G * tiles_n;
-  tm = first + in_group % gm;
-  tn = in_group / gm;
-}
-
 __device__ __forceinline__ void map_tile(int tiles_m, int tiles_n, int& tm, int& tn) {
   map_tile_id(blockIdx.x, tiles_m, tiles_n, tm, tn);
-}
-
-// 8 consecutive elements (one 16-byte bf16 or two 16-byte fp32 accesses when
-// vec8, element by element for a ragged end or unaligned rows).
-__device__ __forceinline__ void load8(const void* p, int64_t off, int dtype, bool vec8, int valid, float* v) {
-  if (vec8 && valid >= 8) {
-    if (dtype == TH_BF16) {
-      const uint4 w = *(const uint4*)((const uint16_t*)p + off);
-      const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        v[2 * q] = __uint_as_float(ws[q] << 16);
-        v[2 * q + 1] = __uint_as_float(ws[q] & 0xffff0000u);
-      }
-    } else {
-      const float4 a = *(const float4*)((const float*)p + off), b = *(const float4*)((const float*)p + off + 4);
-      v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-    }
-    return;
-  }
-#pragma unroll
-  for (int q = 0; q < 8; ++q) v[q] = q < valid ? load_elem(p, off + q, dtype) : 0.f;
-}
-
-__device__ __forceinline__ void store8(void* p, int64_t off, int dtype, bool vec8, int valid, const float* v) {
-  if (vec8 && valid >= 8) {
-    if (dtype == TH_BF16) {
-      uint4 w;
-      w.x = pk_bf16x2(v[0], v[1]);
-      w.y = pk_bf16x2(v[2], v[3]);
-      w.z = pk_bf16x2(v[4], v[5]);
-      w.w = pk_bf16x2(v[6], v[7]);
-      *(uint4*)((uint16_t*)p + off) = w;
-    } else {
-      *(float4*)((float*)p + off) = make_float4(v[0], v[1], v[2], v[3]);
-      *(float4*)((float*)p + off + 4) = make_float4(v[4], v[5], v[6], v[7]);
-    }
-    return;
-  }
-#pragma unroll
-  for (int q = 0; q < 8; ++q)
-    if (q < valid) store_elem(p, off + q, dtype, v[q]);
 }
 
 // One output op over a 16-row slice of the per-wave epilogue (persistent
@@ -231,12 +173,6 @@ __device__ __forceinline__ void epi_slice(const GemmK& p, const EpiOutK& eo, int
   // of them are live (np = 4 with all loaded up front spilled the 8-wave kernel)
   for (int p0 = 0; p0 < np; p0 += 2)
     epi_pair<OP, SUMSQ>(p, eo, o2, wsl, ws, aoff, boff, rsrow, row0, col_w, r_l, c8, np, rp, p0);
-}
-
-// Outputs o and o + 1 compute the same values (same op, operands and column
-// window; only the destination differs).
-__device__ __forceinline__ bool same_values(const EpiOutK& x, const EpiOutK& y) {
-  return x.op == y.op && x.a == y.a && x.b == y.b && x.e == y.e && x.cb == y.cb && x.ce == y.ce;
 }
 
 // Every output op over `rows` staged rows of a whole column tile
@@ -393,16 +329,6 @@ __device__ __forceinline__ float sumsq8_bf16(uint4 w) {
     s += lo * lo + hi * hi;
   }
   return s;
-}
-
-// Sum of squares of an MFMA operand fragment (8 bf16) with v_dot2_f32_bf16:
-// each bf16 product is exact in fp32, accumulation is fp32.
-__device__ __forceinline__ float sumsq8_dot(bf16x8_t v, float acc) {
-  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_shufflevector(v, v, 0, 1), __builtin_shufflevector(v, v, 0, 1), acc, false);
-  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_shufflevector(v, v, 2, 3), __builtin_shufflevector(v, v, 2, 3), acc, false);
-  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_shufflevector(v, v, 4, 5), __builtin_shufflevector(v, v, 4, 5), acc, false);
-  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_shufflevector(v, v, 6, 7), __builtin_shufflevector(v, v, 6, 7), acc, false);
-  return acc;
 }
 
 // --------------------------------------------------------------- bf16 MFMA
@@ -1602,6 +1528,17 @@ static int choose_bn(int64_t N, int n_acc, int in_dtype) {
   }
 }
 
+// About what the direct loop takes (us) on `tiles` 64-row tiles bnc columns wide and
+// nk 64-deep K steps, to compare with gemm_pp_rows's estimate. Measured: 64 x 256 tiles
+// 0.66 us per step whether 16 or 176 of them run (M = 128 .. 700, N = 4096, K = 512 ..
+// 4096), 64 x 128 tiles 0.43; two workgroups on a CU, up to twice as many tiles, 1.3 and
+// 0.58; narrower tiles are taken as the 128-wide ones.
+static double dl64_us(int64_t tiles, int64_t nk, int bnc, int64_t cus) {
+  const double per1 = bnc > 128 ? 0.66 : 0.43, per2 = bnc > 128 ? 1.3 : 0.58;
+  if (tiles <= cus) return 6 + nk * per1;
+  return 6 + (double)cdiv(tiles, 2 * cus) * nk * per2;
+}
+
 static int64_t packed_kp(int64_t K, int in_dtype) {
   const int64_t a = in_dtype == TH_F32 ? 4 : in_dtype == TH_F8E4M3 ? 32 : 8;  // whole 16-byte loads / 32-K chunks
   return (K + a - 1) / a * a;
@@ -1846,22 +1783,7 @@ extern "C" int th_gemm(const th_gemm_desc* d, void* stream) {
                      aligned(d->ss_parts_out, 16) && aligned(d->gain_out, 16),
                  "th_gemm: gain_out needs ss_parts_out [M, N/256] fp32 (16-byte aligned rows) and an aligned gain");
   }
-  int bn = choose_bn(d->N, d->n_acc, d->in_dtype);
-  // One accumulator over 1024 <= N < 2048 columns: 256 x 256 tiles, one per CU
-  // per wave, when they make whole waves, instead of twice as many 256 x 128
-  // tiles: the same MFMA work per CU for a third less operand traffic per FLOP
-  // (16384 x 1024 x 2048: 87.6 -> 75.1 us). N a multiple of 256 keeps the
-  // packed rhs exactly as packed for 128-column tiles (one accumulator's
-  // packed rows are its columns in order, padded to the tile width).
-  bool wide = false;
-  if (d->in_dtype == TH_BF16 && d->n_acc == 1 && bn == 128 && d->N % 256 == 0 && d->K % 64 == 0) {
-    bool rope = false;
-    for (int o = 0; o < d->n_out; ++o) rope |= d->out[o].op == TH_EPI_ROPE || d->out[o].op == TH_EPI_ROPE_PAIR;
-    const int64_t cus = device_cus() > 0 ? device_cus() : 256;
-    const int64_t t256 = cdiv(d->M, 256) * (d->N / 256);
-    wide = !rope && t256 >= cus && t256 % cus == 0;
-    if (wide) bn = 256;
-  }
+  const int bn = choose_bn(d->N, d->n_acc, d->in_dtype);
   GemmK k{};
   k.A = d->lhs;
   k.lda = d->ld_lhs;
@@ -2009,11 +1931,10 @@ extern "C" int th_gemm(const th_gemm_desc* d, void* stream) {
       default: set_error("th_gemm: no fp32 kernel for tile %d", bnc); return TH_ERR_UNSUPPORTED;
     }
   } else {
-    // Row tile: 256 when that still gives two blocks per CU (or for the whole
-    // waves of 256 x 256 tiles above), 128 when it gives one, else 64 (small
-    // problems need the parallelism more than the reuse).
+    // Row tile: 256 when that still gives two blocks per CU, 128 when it gives one,
+    // else 64 (small problems need the parallelism more than the reuse).
     const int64_t cus = device_cus() > 0 ? device_cus() : 256;
-    int bm = wide || cdiv(d->M, 256) * k.tiles_n >= 2 * cus ? 256 : cdiv(d->M, 128) * k.tiles_n >= cus ? 128 : 64;
+    int bm = cdiv(d->M, 256) * k.tiles_n >= 2 * cus ? 256 : cdiv(d->M, 128) * k.tiles_n >= cus ? 128 : 64;
     const bool big = bm == 256;
     k.tiles_m = (int)cdiv(d->M, bm);
     // Direct-to-LDS main loop: whole 64-wide K tiles, and 32-bit buffer offsets
@@ -2039,6 +1960,20 @@ extern "C" int th_gemm(const th_gemm_desc* d, void* stream) {
     if (k.asplit && d->rs_parts != nullptr) {
       set_error("th_gemm: rs_parts is not implemented with whole-head RoPE on two accumulators");
       return TH_ERR_UNSUPPORTED;
+    }
+    // The ping-pong kernel on 256-column tiles, where it is the faster one. (Narrower
+    // packed tiles of one accumulator are its columns in order, padded to the tile, so
+    // a multiple of 256 columns reads as 256-wide tiles too.)
+    GemmK kp = k;
+    if (d->n_acc == 1 && bn == 128 && d->N % 256 == 0) {
+      kp.bn = 256;
+      kp.tiles_n = (int)(d->N / 256);
+    }
+    if (gemm_pp_fits(kp)) {
+      double t_pp = 0;
+      const int pbm = gemm_pp_rows(kp, cus, &t_pp);
+      if (!direct || bm > 64 || t_pp < dl64_us(k.tiles_m * (int64_t)k.tiles_n, d->K / 64, bnc, cus))
+        return launch_gemm_pp(kp, pbm, s);
     }
     MainLoop ml = MainLoop::staged;
     if (direct) ml = wave_epi ? MainLoop::persistent : MainLoop::direct;
