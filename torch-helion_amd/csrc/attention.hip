@@ -169,8 +169,8 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_bf16_kernel(AttnK p) {
   for (int it = 0; it < ntiles; ++it) {
     const int cur = it & 1;
     // tile it has landed everywhere, and every wave is done with stage cur ^ 1
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
+    wait_vmcnt<0>(); wait_lgkmcnt0();
+    barrier_keep_loads();
     if (it + 1 < ntiles) issue(it + 1, cur ^ 1);
     const int k0 = it * BKV;
     const bool active = !p.causal || k0 <= q0w + 31 + p.off;
@@ -198,23 +198,28 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_bf16_kernel(AttnK p) {
       // below 2^8 and the O rescale is skipped while no lane of the wave moves.
       const float c = p.scale_log2;
       const bool need_mask = (k0 + BKV > p.Skv) || (p.causal && k0 + BKV - 1 > q0w + p.off);
-      float mloc = -INFINITY;
       if (need_mask) {
+        // last visible key of this lane's query, from its first key of the tile
+        const int lim = (p.causal ? min(p.Skv - 1, qrow + p.off) : p.Skv - 1) - k0 - 4 * hl;
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int kv = k0 + 32 * t + 8 * (r >> 2) + 4 * hl + (r & 3);
-            if (kv >= p.Skv || (p.causal && kv > qrow + p.off)) s[t][r] = -INFINITY;
-            mloc = fmaxf(mloc, s[t][r]);
-          }
-      } else {
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) mloc = fmaxf(mloc, s[t][r]);
+          for (int r = 0; r < 16; ++r)
+            if (32 * t + 8 * (r >> 2) + (r & 3) > lim) s[t][r] = -INFINITY;
       }
-      mloc = fmaxf(mloc, __shfl_xor(mloc, 32)) * c;
+      // four chains each for the maximum (v_max3) and the sum: one chain of 32 waits for
+      // every result before the next
+      float mx[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; r += 2) mx[(r >> 1) & 3] = fmaxf(fmaxf(mx[(r >> 1) & 3], s[t][r]), s[t][r + 1]);
+      float mloc = fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3]));
+      {
+        // the other half's maximum by a register exchange, not through the LDS crossbar
+        const auto w = __builtin_amdgcn_permlane32_swap(__float_as_uint(mloc), __float_as_uint(mloc), false, false);
+        mloc = fmaxf(__uint_as_float(w[0]), __uint_as_float(w[1])) * c;
+      }
       const bool move = mloc > m_run + 8.f;
       float alpha = 1.f;
       if (move) {
@@ -222,16 +227,16 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_bf16_kernel(AttnK p) {
         m_run = mloc;
       }
       const float nm = m_run == -INFINITY ? 0.f : -m_run;
-      float lsum = 0.f;
+      float ls[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const float ex = __builtin_amdgcn_exp2f(fmaf(s[t][r], c, nm));
           s[t][r] = ex;
-          lsum += ex;
+          ls[r & 3] += ex;
         }
-      l_run = l_run * alpha + lsum;
+      l_run = l_run * alpha + ((ls[0] + ls[1]) + (ls[2] + ls[3]));
       if (__any(move)) {
 #pragma unroll
         for (int t = 0; t < NDT; ++t)
