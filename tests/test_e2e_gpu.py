@@ -614,3 +614,29 @@ def test_buffer_reuse_is_bit_exact(gpu, tmp_path, norm_gain):
                 torch.cuda.synchronize()
                 assert torch.equal(dp.outputs(fp32=True)[0], outs[True])
     assert torch.equal(outs[True], outs[False])
+
+
+@pytest.mark.parametrize("heads,kv_heads,seq", [(8, 4, 200), (16, 8, 129)])
+def test_llama_rotary_projections_merged(gpu, heads, kv_heads, seq, tmp_path):
+    """q, k and v of a grouped-query bf16 block as one launch (heads of 128 and 64) against two launches."""
+    from targets.llama_block import LlamaBlockConfig, build_llama_block
+    from torch_helion import CompileConfig, compile_model
+
+    cfg = LlamaBlockConfig(batch=2, seq=seq, hidden=1024, heads=heads, kv_heads=kv_heads, intermediate=512, causal=True,
+                           dtype=torch.bfloat16)
+    model = build_llama_block(cfg, seed=3)
+    x = model.example_inputs(seed=3)
+    outs = []
+    for merge in (None, False):
+        res = compile_model(model, x, CompileConfig(run_name=f"rotary_{merge}", results_dir=tmp_path, device_check=False,
+                                                    reference_check=False, verify_passes=False, merge_siblings=merge))
+        outs.append(res.run(*x)[0].clone())
+        merged = [l for l in res.device_program.launches if "+" in l.kernel]
+        assert len(merged) == (1 if merge is None else 0)
+    torch.cuda.synchronize()
+    # The products are the same sums in the same order. Two launches may run on another kernel than one, whose
+    # fp32 row sums of squares add up in another order: the row scales then differ by a few 2^-24, which moves a
+    # bf16 rounding here and there (q, k, v, the attention output, the MLP's operands), each by 2^-8 of the value
+    # at most: under 2^-8 of the result's 2-norm even if every value moved.
+    a, b = outs[0].double(), outs[1].double()
+    assert float((a - b).norm() / b.norm()) < 2.0**-8

@@ -1531,11 +1531,12 @@ static int choose_bn(int64_t N, int n_acc, int in_dtype) {
 // About what the direct loop takes (us) on `tiles` 64-row tiles bnc columns wide and
 // nk 64-deep K steps, to compare with gemm_pp_rows's estimate. Measured: 64 x 256 tiles
 // 0.66 us per step whether 16 or 176 of them run (M = 128 .. 700, N = 4096, K = 512 ..
-// 4096), 64 x 128 tiles 0.43; two workgroups on a CU, up to twice as many tiles, 1.3 and
-// 0.58; narrower tiles are taken as the 128-wide ones.
+// 4096), 0.8 - 0.9 on all 256 CUs, 64 x 128 tiles 0.43; two workgroups on a CU, up to
+// twice as many tiles, 1.3 and 0.58; narrower tiles are taken as the 128-wide ones.
 static double dl64_us(int64_t tiles, int64_t nk, int bnc, int64_t cus) {
   const double per1 = bnc > 128 ? 0.66 : 0.43, per2 = bnc > 128 ? 1.3 : 0.58;
-  if (tiles <= cus) return 6 + nk * per1;
+  const double crowd = bnc > 128 ? std::max(0.0, (double)tiles / (double)cus - 0.7) * 0.7 : 0.0;
+  if (tiles <= cus) return 6 + nk * (per1 + crowd);
   return 6 + (double)cdiv(tiles, 2 * cus) * nk * per2;
 }
 

@@ -188,8 +188,8 @@ class DeviceProgram:
             groups = {k: v for k, v in groups.items() if k in keep}
             away = {m[0].name for v in groups.values() for m in v[1:]}
         self._merge_groups, self._merged_away = groups, away
-        # (e4m3 decode GEMMs: a few rows against weight streams, one launch always pays)
-        self._fp8_groups = self._plan_fp8_merges(program, self._merged_away) if merge_siblings is not False else {}
+        # (rotary siblings and e4m3 decode GEMMs: one launch always pays, see _plan_rotary_merges)
+        self._rotary_groups = self._plan_rotary_merges(program, self._merged_away) if merge_siblings is not False else {}
         # scans whose only reader normalises them with a gain: the scan applies it (_plan_norm_folds)
         self._rs_parts: dict[tuple, torch.Tensor] = {}
         self._norm_folds = self._plan_norm_folds(program)
@@ -201,7 +201,7 @@ class DeviceProgram:
             if self.reuse:
                 self._pool.release_before(i)
                 self._bind_outputs(k)
-                for m in (self._merge_groups.get(k.name) or self._fp8_groups.get(k.name) or [])[1:]:
+                for m in (self._merge_groups.get(k.name) or self._rotary_groups.get(k.name) or [])[1:]:
                     self._bind_outputs(m[0])
             if k.name in self._merged_away:
                 continue
@@ -212,9 +212,9 @@ class DeviceProgram:
                 continue  # runs with its group, at the group's last member
             if k.name in self._merge_groups:
                 self.launches.extend(self._lower_gemm_merged(self._merge_groups[k.name]))
-            elif k.name in self._fp8_groups:
-                members = [m[0] for m in self._fp8_groups[k.name]]
-                merged = self._lower_fp8_merged(members)
+            elif k.name in self._rotary_groups:
+                members = [m[0] for m in self._rotary_groups[k.name]]
+                merged = self._lower_rotary_merged(members)
                 if merged is None:  # the parts disagree: each member at the leader's position
                     merged = [x for m in members for x in self._lower(m)]
                 self.launches.extend(merged)
@@ -774,7 +774,7 @@ class DeviceProgram:
             if len(rd) != 1 or rd[0][0].kind != "gemm" or rd[0][1].role != "lhs" or not rd[0][0].gemms:
                 continue
             g = rd[0][0]
-            if g.name in self._merge_groups or g.name in self._merged_away or g.name in self._fp8_groups:
+            if g.name in self._merge_groups or g.name in self._merged_away or g.name in self._rotary_groups:
                 continue
             plan = match_epilogue(g)
             if not plan.fused or plan.rscale is None or any(o.rope is not None for o in plan.outs):
@@ -808,7 +808,7 @@ class DeviceProgram:
 
         def alone(k: KernelSpec) -> bool:
             return k.name not in self._merge_groups and k.name not in self._merged_away and not any(
-                k.name == m[0].name for v in self._fp8_groups.values() for m in v)
+                k.name == m[0].name for v in self._rotary_groups.values() for m in v)
 
         taken: set[str] = set()
         for g in program.kernels:
@@ -977,44 +977,60 @@ class DeviceProgram:
         launch = Launch("+".join(names), "gemm", run, "th_gemm", info)
         return [norm_launch, launch] if norm_launch is not None else [launch]
 
-    # e4m3 sibling merge (decode programs): GEMM kernels with e4m3 weights that
-    # read the same lhs (q and k|v of the decode step) run as ONE th_gemm over
-    # the concatenated weights and scales, each output on its own column window
-    # (fused RoPE included: a head never straddles two windows), with one
-    # activation-gain pre-pass and one reduce pass instead of one per kernel.
-    def _plan_fp8_merges(self, program: Program, away: set[str]):
+    # Rotary sibling merge: GEMM kernels that read the same lhs (q and k|v of a
+    # block) run as ONE th_gemm over the concatenated weights, each output on its
+    # own column window (fused RoPE included: a head never straddles two windows).
+    # e4m3 weights (decode programs): one activation-gain pre-pass and one reduce
+    # pass instead of one per kernel. bf16 weights: q and k|v of a grouped-query
+    # block alone leave half the CUs idle at a few thousand rows (2000 rows, K =
+    # 2048: q 37 us on 128 .. 256 tiles, k|v 34 us on 64; together on 192 tiles
+    # 33 us) and fill the same rounds of tiles together that they fill apart at
+    # many rows.
+    def _plan_rotary_merges(self, program: Program, away: set[str]):
         produced_at = {o.tensor: i for i, k in enumerate(program.kernels) for o in k.outputs}
 
         def key(k: KernelSpec):
             if k.kind != "gemm" or not k.gemms:
                 return None
-            if any(self.program.tensors[k.arg(g.rhs).tensor].dtype != "float8_e4m3fn" for g in k.gemms):
+            ts = [self.program.tensors[k.arg(g.rhs).tensor].dtype for g in k.gemms]
+            if any(t == "float8_e4m3fn" for t in ts):
+                if any(t != "float8_e4m3fn" for t in ts):
+                    return None
+                return ("e4m3", k.arg("lhs").tensor, k.k_extent, k.grid["rows"])
+            # bf16: the rotary projections of one input (parameter weights, no norm gain to take back out)
+            if self.fold_sources or self.program.tensors[k.arg("lhs").tensor].dtype != "bfloat16":
                 return None
-            return (k.arg("lhs").tensor, k.k_extent, k.grid["rows"])
+            if any(k.arg(g.rhs).tensor not in program.params for g in k.gemms) or k.grid["cols"] % 8:
+                return None
+            return ("bf16", k.arg("lhs").tensor, k.k_extent, k.grid["rows"])
+
+        def rotary(k: KernelSpec) -> bool:
+            plan = match_epilogue(k)
+            return plan.fused and any(o.rope is not None for o in plan.outs)
 
         groups: dict[str, list] = {}
         for i, k in enumerate(program.kernels):
             ki = key(k)
-            if ki is None or k.name in away:
+            if ki is None or k.name in away or k.name in self._merge_groups:
                 continue
             members = [k]
             for j in range(i + 1, len(program.kernels)):
                 k2 = program.kernels[j]
-                if k2.name in away or key(k2) != ki:
+                if k2.name in away or k2.name in self._merge_groups or key(k2) != ki:
                     continue
                 # every other operand exists before the leader runs (params, program
                 # inputs and constants, or an earlier kernel's output)
                 ins = {a.tensor for a in k2.args if a.name != "lhs"}
                 if all(produced_at.get(t, -1) < i for t in ins):
                     members.append(k2)
-            if len(members) > 1:
+            if len(members) > 1 and (ki[0] == "e4m3" or any(rotary(m) for m in members)):
                 groups[k.name] = [(m, None, None) for m in members]
                 away.update(m.name for m in members[1:])
         return groups
 
-    def _lower_fp8_merged(self, members: list[KernelSpec]) -> list[Launch] | None:
-        """One th_gemm for these e4m3 kernels, or None when their parts disagree
-        (lhs, row scale, gain, RoPE tables) or an output needs a second accumulator
+    def _lower_rotary_merged(self, members: list[KernelSpec]) -> list[Launch] | None:
+        """One th_gemm for these kernels, or None when their parts disagree (weight type,
+        lhs, row scale, gain, RoPE tables) or an output needs a second accumulator
         or an extra operand."""
         parts = []
         for spec in members:
@@ -1025,8 +1041,9 @@ class DeviceProgram:
             parts.append((spec, col[0]))
         p0 = parts[0][1]
         rope = next((pt["rope"] for _, pt in parts if pt["rope"] is not None), None)
+        fp8 = p0["fp8"]
         for spec, pt in parts:
-            if not pt["fp8"] or pt["lhs"] is not p0["lhs"] or pt["extras"] or pt["norm"] is not None:
+            if pt["fp8"] != fp8 or pt["lhs"] is not p0["lhs"] or pt["extras"] or pt["norm"] is not None:
                 return None
             if (pt["T"], pt["K"], pt["sumsq"], pt["inv_k"], pt["eps"]) != (p0["T"], p0["K"], p0["sumsq"], p0["inv_k"], p0["eps"]):
                 return None
@@ -1048,9 +1065,10 @@ class DeviceProgram:
         n_tot = 0
         for spec, pt in parts:
             win = {}
-            for slot, (t, st) in enumerate(zip(pt["rhs"], pt["scales"])):
-                ws_.append(self.buffers[t].view(torch.uint8))
-                scales.append(self.buffers[st].float().reshape(-1))
+            for slot, (t, st) in enumerate(zip(pt["rhs"], pt["scales"] if fp8 else pt["rhs"])):
+                ws_.append(self.buffers[t].view(torch.uint8) if fp8 else self.buffers[t].to(torch.bfloat16))
+                if fp8:
+                    scales.append(self.buffers[st].float().reshape(-1))
                 win[slot] = (n_tot, n_tot + pt["N"])
                 n_tot += pt["N"]
             for e in pt["epi"]:
@@ -1064,15 +1082,22 @@ class DeviceProgram:
             return None
         if rope is not None and n_tot % rope[3]:
             return None
-        packed = ops.pack_rhs([torch.cat(ws_, dim=1).view(_FP8).contiguous()], _FP8)
-        scale = torch.cat(scales).reshape(1, -1).contiguous()
-        ws = self._workspace(max(ops.gemm_workspace_bytes(T, n_tot, K, 1, _FP8), 16), torch.uint8)
+        if not fp8 and (rope is None or rope[3] < 64 or 256 % rope[3] or n_tot % 256 or n_tot < 2048):
+            return None  # (256-column tiles of whole heads)
         names = [spec.name for spec, _ in parts]
         info = {"n_acc": 1, "merged": names, "cols": n_tot, "ops": [x.op for x in epi], "rscale": p0["sumsq"],
-                "rope_fused": rope is not None, "weights": "float8_e4m3fn", "lhs_gain": p0["lhs_gain"] is not None}
+                "rope_fused": rope is not None}
+        dt = _FP8 if fp8 else torch.bfloat16
+        cat = torch.cat(ws_, dim=1)
+        packed = ops.pack_rhs([(cat.view(_FP8) if fp8 else cat).contiguous()], dt)
+        extra: dict[str, Any] = {}
+        if fp8:
+            extra = dict(rhs_scale=torch.cat(scales).reshape(1, -1).contiguous(),
+                         workspace=self._workspace(max(ops.gemm_workspace_bytes(T, n_tot, K, 1, _FP8), 16), torch.uint8))
+            info.update({"weights": "float8_e4m3fn", "lhs_gain": p0["lhs_gain"] is not None})
         lhs, gain = p0["lhs"], p0["lhs_gain"]
         kw = dict(sumsq=p0["sumsq"], rscale_mask=1 if p0["mask"] else 0, inv_k=p0["inv_k"], eps=p0["eps"],
-                  in_dtype=_FP8, rhs_scale=scale, workspace=ws)
+                  in_dtype=dt, **extra)
         if gain is not None:
             kw["lhs_gain"] = gain
 
