@@ -786,13 +786,17 @@ __global__ void __launch_bounds__(256) gemm_fp8_reduce_kernel(Fp8K p) {
 // sums in split order, 4-wide stores. S > 0: exactly S splits, every partial
 // the thread adds (its columns, the RoPE partner's, the row's sums of squares)
 // loaded before the first is added, with the extras and RoPE tables: one
-// memory round trip. S = 0: any split count, a loop per sum. Requires
+// memory round trip. NA and ROPE bound what is held for that: up to 8 splits two
+// accumulators and their RoPE partners, 9 to 16 one accumulator without (registers).
+// S = 0: any split count, a loop per sum, a few loads at a time: the o and down
+// projections of a small step (8 rows, 2048 columns, 15 and 16 splits) spent 8.8 us
+// in it. Blocks of 64 threads where 256-thread ones would leave CUs idle. Requires
 // N % 4 == 0 and a power-of-two bn (so 4 columns share a tile). With
 // gain_out (N a multiple of 1024, so every wave is whole and inside one row),
 // each wave sums its 256 columns' bf16(v)^2 into ss_parts_out.
-template <int S>
+template <int S, int NA = 2, bool ROPE = true>
 __global__ void __launch_bounds__(256) gemm_fp8_reduce4_kernel(Fp8K p) {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t nq = p.N >> 2;
   if (idx >= p.M * nq) return;
   const int64_t m = idx / nq, n4 = (idx - m * nq) << 2;
@@ -867,14 +871,14 @@ __global__ void __launch_bounds__(256) gemm_fp8_reduce4_kernel(Fp8K p) {
         for (int sp = 0; sp < S; ++sp) ps[sp] = p.sumsq_part[(int64_t)sp * p.M + m];
       }
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
+      for (int i = 0; i < NA; ++i) {
         if (i < na) {
           const float* q = part_ptr(i, n4);
 #pragma unroll
           for (int sp = 0; sp < S; ++sp) pa[i][sp] = *(const float4*)(q + sp * plane);
           sa[i] = *(const float4*)(p.scale + (int64_t)i * p.N + n4);
         }
-        if (i < na && rope_acc[i]) {
+        if (ROPE && i < na && rope_acc[i]) {
           const float* q = part_ptr(i, pn);
 #pragma unroll
           for (int sp = 0; sp < S; ++sp) pr[i][sp] = *(const float4*)(q + sp * plane);
@@ -1011,16 +1015,27 @@ int launch_gemm_fp8(const GemmK& k, int64_t Npk, const float* scale, float* ws, 
     TH_CHECK_LAUNCH();
     if (!p.fused) {
       if (vec) {
-        const dim3 gr((unsigned)cdiv(k.M * (k.N / 4), 256));
-        switch (p.splits) {
+        const int64_t cus = device_cus() > 0 ? device_cus() : 256, work = k.M * (k.N / 4);
+        const int nt = cdiv(work, 256) < cus ? 64 : 256;
+        const dim3 gr((unsigned)cdiv(work, nt)), bl((unsigned)nt);
+        bool plain = k.n_acc == 1;  // one accumulator, no RoPE partner
+        for (int o = 0; o < k.n_out; ++o) plain &= k.out[o].op != TH_EPI_ROPE;
+        switch (p.splits > 8 && !plain ? 0 : p.splits) {
 #define TH_FP8_RED4(S_) \
   case S_:              \
-    hipLaunchKernelGGL(gemm_fp8_reduce4_kernel<S_>, gr, dim3(256), 0, stream, p); \
+    hipLaunchKernelGGL(gemm_fp8_reduce4_kernel<S_>, gr, bl, 0, stream, p); \
+    break;
+#define TH_FP8_RED4P(S_) \
+  case S_:               \
+    hipLaunchKernelGGL((gemm_fp8_reduce4_kernel<S_, 1, false>), gr, bl, 0, stream, p); \
     break;
           TH_FP8_RED4(2) TH_FP8_RED4(3) TH_FP8_RED4(4) TH_FP8_RED4(5) TH_FP8_RED4(6) TH_FP8_RED4(7) TH_FP8_RED4(8)
+          TH_FP8_RED4P(9) TH_FP8_RED4P(10) TH_FP8_RED4P(11) TH_FP8_RED4P(12) TH_FP8_RED4P(13) TH_FP8_RED4P(14)
+          TH_FP8_RED4P(15) TH_FP8_RED4P(16)
 #undef TH_FP8_RED4
+#undef TH_FP8_RED4P
           default:
-            hipLaunchKernelGGL(gemm_fp8_reduce4_kernel<0>, gr, dim3(256), 0, stream, p);
+            hipLaunchKernelGGL(gemm_fp8_reduce4_kernel<0>, gr, bl, 0, stream, p);
         }
       }
       else
