@@ -786,15 +786,11 @@ __global__ void __launch_bounds__(256) gemm_fp8_reduce_kernel(Fp8K p) {
 // sums in split order, 4-wide stores. S > 0: exactly S splits, every partial
 // the thread adds (its columns, the RoPE partner's, the row's sums of squares)
 // loaded before the first is added, with the extras and RoPE tables: one
-// memory round trip. NA and ROPE bound what is held for that: up to 8 splits two
-// accumulators and their RoPE partners, 9 to 16 one accumulator without (registers).
-// S = 0: any split count, a loop per sum, a few loads at a time: the o and down
-// projections of a small step (8 rows, 2048 columns, 15 and 16 splits) spent 8.8 us
-// in it. Blocks of 64 threads where 256-thread ones would leave CUs idle. Requires
-// N % 4 == 0 and a power-of-two bn (so 4 columns share a tile). With
+// memory round trip. S = 0: any split count, a loop per sum. Blocks of 64 threads
+// where 256-thread ones would leave CUs idle. Requires N % 4 == 0 and a power-of-two bn (so 4 columns share a tile). With
 // gain_out (N a multiple of 1024, so every wave is whole and inside one row),
 // each wave sums its 256 columns' bf16(v)^2 into ss_parts_out.
-template <int S, int NA = 2, bool ROPE = true>
+template <int S>
 __global__ void __launch_bounds__(256) gemm_fp8_reduce4_kernel(Fp8K p) {
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t nq = p.N >> 2;
@@ -871,14 +867,14 @@ __global__ void __launch_bounds__(256) gemm_fp8_reduce4_kernel(Fp8K p) {
         for (int sp = 0; sp < S; ++sp) ps[sp] = p.sumsq_part[(int64_t)sp * p.M + m];
       }
 #pragma unroll
-      for (int i = 0; i < NA; ++i) {
+      for (int i = 0; i < 2; ++i) {
         if (i < na) {
           const float* q = part_ptr(i, n4);
 #pragma unroll
           for (int sp = 0; sp < S; ++sp) pa[i][sp] = *(const float4*)(q + sp * plane);
           sa[i] = *(const float4*)(p.scale + (int64_t)i * p.N + n4);
         }
-        if (ROPE && i < na && rope_acc[i]) {
+        if (i < na && rope_acc[i]) {
           const float* q = part_ptr(i, pn);
 #pragma unroll
           for (int sp = 0; sp < S; ++sp) pr[i][sp] = *(const float4*)(q + sp * plane);
@@ -906,6 +902,243 @@ __global__ void __launch_bounds__(256) gemm_fp8_reduce4_kernel(Fp8K p) {
       return row_scale(ss);
     };
     store_ss_part(fp8_emit4(p, m, n4, rrf, sum4, gather));
+  }
+}
+
+// ------------------------------------------------ the decode step's reductions
+// gemm_fp8_reduce4_kernel for the three output forms a decode step has, each in a
+// kernel of its own with no more code and arguments than the form needs. What
+// bounds the reduction of a small step (1 MB of partials and less) is neither
+// bandwidth nor the round trip but its first execution after other kernels: the
+// general one, with six unrolled outputs of eight ops, takes 6.2 - 7.8 us between a
+// step's kernels and 2.9 - 4.2 us when it alone repeats.
+//   RED_ADD   one accumulator, every output its sum plus the same operand, all
+//             columns (o and down projections), one of them through gain_out
+//   RED_GLU   two accumulators, one SWIGLU output
+//   RED_ROPE  one accumulator, ROPE and plain outputs on column windows
+enum { RED_ADD = 0, RED_GLU = 1, RED_ROPE = 2 };
+
+struct RedOut {
+  void* p;
+  int64_t ld;
+  int dtype, op, cb, ce;
+};
+
+struct RedK {
+  const float* part;
+  const float* scale;
+  const float* ssq;  // [splits][M] partial row sums of squares, or
+  const float* rsp;  // [M][n_rsp] (row stride ld_rsp) the producer's parts
+  int64_t ld_rsp, plane, npk, ldx;
+  int M, N, sh, n_rsp, n_out, gidx, hd, period;
+  unsigned mask;
+  int ga, gb, xdt;
+  float inv_k, eps;
+  float* sumsq_out;
+  const void* x;
+  const float* rcos;
+  const float* rsin;
+  const float* gain;
+  float* gss;
+  int64_t ld_gss;
+  RedOut out[3];
+};
+
+template <int KIND, int S>
+__global__ void __launch_bounds__(256) gemm_fp8_red_kernel(RedK p) {
+  const int nq = p.N >> 2;
+  const int idx = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (idx >= p.M * nq) return;
+  const int m = idx / nq, n4 = (idx - m * nq) << 2;
+  constexpr int NA = KIND == RED_GLU ? 2 : 1;
+  // accumulator i at columns nn .. nn + 3: every split's partial sums
+  auto part_ptr = [&](int i, int nn) {
+    const int64_t t = nn >> p.sh;
+    const int j = nn & ((1 << p.sh) - 1);
+    return p.part + (int64_t)m * p.npk + ((t * NA + i) << p.sh) + j;
+  };
+  float4 v[NA + (KIND == RED_ROPE)][S], sc[NA + (KIND == RED_ROPE)];
+  int within = 0, pn = n4;
+  bool rope = false;
+  float4 cs = make_float4(0.f, 0.f, 0.f, 0.f), sn = cs, x = cs, gq = cs;
+  if constexpr (KIND == RED_ROPE) {
+    for (int o = 0; o < p.n_out; ++o) rope |= p.out[o].op == TH_EPI_ROPE && n4 >= p.out[o].cb && n4 < p.out[o].ce;
+    within = n4 % p.hd;
+    if (rope) pn = within < (p.hd >> 1) ? n4 + (p.hd >> 1) : n4 - (p.hd >> 1);
+  }
+#pragma unroll
+  for (int i = 0; i < NA; ++i) {
+    const float* q = part_ptr(i, n4);
+#pragma unroll
+    for (int sp = 0; sp < S; ++sp) v[i][sp] = *(const float4*)(q + sp * p.plane);
+    sc[i] = *(const float4*)(p.scale + (int64_t)i * p.N + n4);
+  }
+  if constexpr (KIND == RED_ROPE) {
+    const float* q = part_ptr(0, pn);
+#pragma unroll
+    for (int sp = 0; sp < S; ++sp) v[1][sp] = *(const float4*)(q + sp * p.plane);
+    sc[1] = *(const float4*)(p.scale + pn);
+    const int64_t toff = (int64_t)(m % p.period) * p.hd + within;
+    cs = *(const float4*)(p.rcos + toff);
+    sn = *(const float4*)(p.rsin + toff);
+  }
+  if constexpr (KIND == RED_ADD) {
+    x = load4(p.x, (int64_t)m * p.ldx + n4, p.xdt, true, 4);
+    if (p.gain != nullptr) gq = *(const float4*)(p.gain + n4);
+  }
+  float rr = 1.f;
+  if constexpr (KIND != RED_ADD) {
+    float ps[S];
+    if (p.ssq != nullptr) {
+#pragma unroll
+      for (int sp = 0; sp < S; ++sp) ps[sp] = p.ssq[sp * p.M + m];
+    }
+    if (p.ssq != nullptr || p.rsp != nullptr) {
+      float ss;
+      if (p.rsp != nullptr) {
+        ss = row_parts_sum((const float4*)(p.rsp + (int64_t)m * p.ld_rsp), p.n_rsp >> 2);
+      } else {
+        ss = ps[0];
+#pragma unroll
+        for (int sp = 1; sp < S; ++sp) ss += ps[sp];
+      }
+      if (p.sumsq_out && n4 == 0) p.sumsq_out[m] = ss;
+      rr = rsqrtf(ss * p.inv_k + p.eps);
+    }
+  }
+  auto sum = [&](int i) {
+    float4 a = v[i][0];
+#pragma unroll
+    for (int sp = 1; sp < S; ++sp) {
+      a.x += v[i][sp].x; a.y += v[i][sp].y; a.z += v[i][sp].z; a.w += v[i][sp].w;
+    }
+    return make_float4(a.x * sc[i].x, a.y * sc[i].y, a.z * sc[i].z, a.w * sc[i].w);
+  };
+  auto scl = [](float4 a, float f) { return make_float4(a.x * f, a.y * f, a.z * f, a.w * f); };
+  if constexpr (KIND == RED_GLU) {
+    const float4 c0 = sum(0), c1 = sum(1);
+    float4 a = p.ga ? c1 : c0, b = p.gb ? c1 : c0;
+    if ((p.mask >> p.ga) & 1u) a = scl(a, rr);
+    if ((p.mask >> p.gb) & 1u) b = scl(b, rr);
+    const float4 r = make_float4(a.x * sigmoidf_(a.x) * b.x, a.y * sigmoidf_(a.y) * b.y, a.z * sigmoidf_(a.z) * b.z,
+                                 a.w * sigmoidf_(a.w) * b.w);
+    const RedOut& eo = p.out[0];
+    if (n4 >= eo.cb && n4 < eo.ce) store4(eo.p, (int64_t)m * eo.ld + (n4 - eo.cb), eo.dtype, true, 4, r);
+  } else if constexpr (KIND == RED_ROPE) {
+    float4 a = sum(0);
+    if (p.mask & 1u) a = scl(a, rr);
+    float4 w = a;
+    if (rope) {
+      const float sg = within < (p.hd >> 1) ? -1.f : 1.f;
+      const float4 r = scl(sum(1), p.mask & 1u ? sg * rr : sg);
+      w = make_float4(a.x * cs.x + r.x * sn.x, a.y * cs.y + r.y * sn.y, a.z * cs.z + r.z * sn.z, a.w * cs.w + r.w * sn.w);
+    }
+#pragma unroll 1
+    for (int o = 0; o < p.n_out; ++o) {
+      const RedOut& eo = p.out[o];
+      if (n4 >= eo.cb && n4 < eo.ce)
+        store4(eo.p, (int64_t)m * eo.ld + (n4 - eo.cb), eo.dtype, true, 4, eo.op == TH_EPI_ROPE ? w : a);
+    }
+  } else {
+    // (the scaled sum rounded before the addition, as in the general kernel and in the
+    // tiles that the main kernel finishes)
+#pragma clang fp contract(off)
+    const float4 a = sum(0);
+    const float4 r = make_float4(a.x + x.x, a.y + x.y, a.z + x.z, a.w + x.w);
+    float ssg = 0.f;
+#pragma unroll 1
+    for (int o = 0; o < p.n_out; ++o) {
+      const RedOut& eo = p.out[o];
+      float4 w = r;
+      if (p.gain != nullptr && o == p.gidx) {
+        // the value the output would hold, then times the next RMSNorm's gain
+        auto rb = [](float f) { return __uint_as_float((uint32_t)f32_to_bf16(f) << 16); };
+        const float4 t = make_float4(rb(r.x), rb(r.y), rb(r.z), rb(r.w));
+        ssg = ((t.x * t.x + t.y * t.y) + t.z * t.z) + t.w * t.w;
+        w = make_float4(t.x * gq.x, t.y * gq.y, t.z * gq.z, t.w * gq.w);
+      }
+      store4(eo.p, (int64_t)m * eo.ld + n4, eo.dtype, true, 4, w);
+    }
+    if (p.gain != nullptr) {  // (N a multiple of 1024: a wave is whole and inside one row)
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) ssg += __shfl_xor(ssg, off);
+      if ((threadIdx.x & 63) == 0) p.gss[(int64_t)m * p.ld_gss + (n4 >> 8)] = ssg;
+    }
+  }
+}
+
+// The form of these outputs (RED_*), or -1 for the general kernel.
+static int fp8_red_kind(const Fp8K& p) {
+  const GemmK& g = p.k;
+  if (g.n_out > 3 || p.M * (p.N >> 2) >= ((int64_t)1 << 31) || p.N % 4 != 0) return -1;
+  bool add = g.n_acc == 1 && !g.sumsq, glu = g.n_acc == 2 && g.n_out == 1, rope = g.n_acc == 1, any_rope = false;
+  for (int o = 0; o < g.n_out; ++o) {
+    const EpiOutK& eo = g.out[o];
+    if (!eo.vec || eo.ce % 4 != 0) return -1;
+    add &= eo.op == TH_EPI_ADD && eo.e == g.out[0].e && eo.cb == 0 && eo.ce == (int)p.N && g.extra_vec[eo.e >= 0 ? eo.e : 0];
+    glu &= eo.op == TH_EPI_SWIGLU;
+    rope &= (eo.op == TH_EPI_ROPE && g.hd % 8 == 0) || eo.op == TH_EPI_ACC;
+    any_rope |= eo.op == TH_EPI_ROPE;
+  }
+  if (add && p.splits <= 16) return RED_ADD;
+  if (p.splits > 8 || g.gain_out != nullptr) return -1;
+  return glu ? RED_GLU : rope && any_rope ? RED_ROPE : -1;
+}
+
+static void launch_fp8_red(const Fp8K& p, int kind, int nt, hipStream_t s) {
+  const GemmK& g = p.k;
+  RedK r{};
+  r.part = p.part;
+  r.scale = p.scale;
+  r.ssq = g.sumsq && p.ss_pre != 2 ? p.sumsq_part : nullptr;
+  r.rsp = g.sumsq && p.ss_pre == 2 ? g.rs_parts : nullptr;
+  r.ld_rsp = g.ld_rs_parts;
+  r.n_rsp = g.n_rs_parts;
+  r.plane = p.M * p.Npk;
+  r.npk = p.Npk;
+  r.M = (int)p.M;
+  r.N = (int)p.N;
+  r.sh = __builtin_ctz((unsigned)p.bn);
+  r.n_out = g.n_out;
+  r.mask = g.rscale_mask;
+  r.inv_k = g.inv_k;
+  r.eps = g.eps;
+  r.sumsq_out = g.sumsq_out;
+  r.rcos = g.rcos;
+  r.rsin = g.rsin;
+  r.hd = g.hd;
+  r.period = g.period;
+  r.gain = g.gain_out;
+  r.gss = g.ss_parts_out;
+  r.ld_gss = g.ld_ss_parts_out;
+  r.gidx = g.gain_index;
+  r.ga = g.out[0].a;
+  r.gb = g.out[0].b;
+  if (kind == RED_ADD) {
+    r.x = g.extra[g.out[0].e];
+    r.ldx = g.ld_extra[g.out[0].e];
+    r.xdt = g.extra_dtype[g.out[0].e];
+  }
+  for (int o = 0; o < g.n_out; ++o)
+    r.out[o] = {g.out[o].ptr, g.out[o].ld, g.out[o].dtype, g.out[o].op, g.out[o].cb, g.out[o].ce};
+  const dim3 gr((unsigned)cdiv(p.M * (p.N / 4), nt)), bl((unsigned)nt);
+  auto go = [&](auto sc) {
+    constexpr int S = decltype(sc)::value;
+    if (kind == RED_ADD) {
+      hipLaunchKernelGGL((gemm_fp8_red_kernel<RED_ADD, S>), gr, bl, 0, s, r);
+    } else if constexpr (S <= 8) {
+      if (kind == RED_GLU)
+        hipLaunchKernelGGL((gemm_fp8_red_kernel<RED_GLU, S>), gr, bl, 0, s, r);
+      else
+        hipLaunchKernelGGL((gemm_fp8_red_kernel<RED_ROPE, S>), gr, bl, 0, s, r);
+    }
+  };
+  switch (p.splits) {
+#define TH_RED_S(S_) \
+  case S_: go(std::integral_constant<int, S_>{}); break;
+    TH_RED_S(1) TH_RED_S(2) TH_RED_S(3) TH_RED_S(4) TH_RED_S(5) TH_RED_S(6) TH_RED_S(7) TH_RED_S(8)
+    TH_RED_S(9) TH_RED_S(10) TH_RED_S(11) TH_RED_S(12) TH_RED_S(13) TH_RED_S(14) TH_RED_S(15) TH_RED_S(16)
+#undef TH_RED_S
   }
 }
 
@@ -1018,22 +1251,19 @@ int launch_gemm_fp8(const GemmK& k, int64_t Npk, const float* scale, float* ws, 
         const int64_t cus = device_cus() > 0 ? device_cus() : 256, work = k.M * (k.N / 4);
         const int nt = cdiv(work, 256) < cus ? 64 : 256;
         const dim3 gr((unsigned)cdiv(work, nt)), bl((unsigned)nt);
-        bool plain = k.n_acc == 1;  // one accumulator, no RoPE partner
-        for (int o = 0; o < k.n_out; ++o) plain &= k.out[o].op != TH_EPI_ROPE;
-        switch (p.splits > 8 && !plain ? 0 : p.splits) {
+        const int kind = fp8_red_kind(p);
+        if (kind >= 0) {
+          launch_fp8_red(p, kind, nt, stream);
+          TH_CHECK_LAUNCH();
+          return TH_OK;
+        }
+        switch (p.splits) {
 #define TH_FP8_RED4(S_) \
   case S_:              \
     hipLaunchKernelGGL(gemm_fp8_reduce4_kernel<S_>, gr, bl, 0, stream, p); \
     break;
-#define TH_FP8_RED4P(S_) \
-  case S_:               \
-    hipLaunchKernelGGL((gemm_fp8_reduce4_kernel<S_, 1, false>), gr, bl, 0, stream, p); \
-    break;
           TH_FP8_RED4(2) TH_FP8_RED4(3) TH_FP8_RED4(4) TH_FP8_RED4(5) TH_FP8_RED4(6) TH_FP8_RED4(7) TH_FP8_RED4(8)
-          TH_FP8_RED4P(9) TH_FP8_RED4P(10) TH_FP8_RED4P(11) TH_FP8_RED4P(12) TH_FP8_RED4P(13) TH_FP8_RED4P(14)
-          TH_FP8_RED4P(15) TH_FP8_RED4P(16)
 #undef TH_FP8_RED4
-#undef TH_FP8_RED4P
           default:
             hipLaunchKernelGGL(gemm_fp8_reduce4_kernel<0>, gr, bl, 0, stream, p);
         }

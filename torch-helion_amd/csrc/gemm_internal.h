@@ -61,10 +61,7 @@ struct GemmK {
 // first addition (indices clamped, additions past the end selected away: no
 // branch for the compiler to put a wait into), so a row costs one memory
 // round trip per 32 parts instead of one per 4.
-__device__ __forceinline__ float row_sumsq(const GemmK& p, int64_t row, float own) {
-  if (p.rs_parts == nullptr) return own;
-  const float4* q = (const float4*)(p.rs_parts + (row < p.M ? row : p.M - 1) * p.ld_rs_parts);
-  const int n4 = p.n_rs_parts >> 2;
+__device__ __forceinline__ float row_parts_sum(const float4* q, int n4) {
   float v = 0.f;
   for (int i0 = 0; i0 < n4; i0 += 8) {
     float4 f[8];
@@ -80,6 +77,11 @@ __device__ __forceinline__ float row_sumsq(const GemmK& p, int64_t row, float ow
     }
   }
   return v;
+}
+
+__device__ __forceinline__ float row_sumsq(const GemmK& p, int64_t row, float own) {
+  if (p.rs_parts == nullptr) return own;
+  return row_parts_sum((const float4*)(p.rs_parts + (row < p.M ? row : p.M - 1) * p.ld_rs_parts), p.n_rs_parts >> 2);
 }
 
 // fp8-weight path (gemm_fp8.hip)
