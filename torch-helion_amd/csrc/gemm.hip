@@ -1297,10 +1297,15 @@ __global__ void __launch_bounds__(1024, 1) gemm_f32_sk_kernel(GemmK p) {
 
 // ------------------------- fp32 MFMA, small grids with a workspace (split-K over workgroups)
 // Pass 1 (gemm_f32_ksp_kernel): workgroup (tile, g) multiplies 32 rows x BNC
-// packed columns over K slice g, one wave per 32 x 32 subtile, with the same
-// operand layout and wave-private LDS ring as gemm_f32_sk_kernel, and stores its
+// packed columns over K slice g, one wave per 32 x 32 subtile, and stores its
 // partial tile to part[g][row][column] (rows of the padded row count Mp); the
 // column-0 workgroups also store the slice's row sums of squares ssq[g][row].
+// What bounds it is memory latency: a slice is a few KB per row. The workgroup
+// streams 32-wide K steps of its 32 + BNC rows (whole 128-byte lines, the lhs rows
+// once for all waves) through up to 80 KiB of LDS stages, two workgroups per CU,
+// so that most of a slice is in flight at once. (Wave-private rings of 8-wide steps,
+// 32 bytes of a line at a time and the lhs rows once per wave: gate/up 128 x 2 * 1376
+// x 512 15.4 us, now 11.1 us; the 128 x 512 fp32 block 72.4 -> 64.9 us.)
 // Pass 2 (gemm_f32_ksr_kernel): one workgroup per 8 (or 2) rows x BNC columns sums the
 // KSG partials in slice order (deterministic) into an LDS slab and runs the
 // slab epilogue. Enough pass-1 workgroups to cover the GPU (about one per CU)
@@ -1316,8 +1321,13 @@ struct F32Ksp {
 template <int BNC>
 __global__ void __launch_bounds__(BNC * 2) gemm_f32_ksp_kernel(F32Ksp q) {
 #if defined(__HIP_DEVICE_COMPILE__)  // gfx950 LDS-load instructions exist only in the device pass
-  constexpr int NSUB = BNC / 32, STEP = 2048, PD = 4;
-  __shared__ __attribute__((aligned(16))) char smem[NSUB * PD * STEP];
+  constexpr int NSUB = BNC / 32;             // waves
+  constexpr int STAGE = (32 + BNC) * 128;    // one K step: 32 floats of every row
+  constexpr int NST = 81920 / STAGE < 8 ? 81920 / STAGE : 8;
+  constexpr int NLD = (32 + BNC) / 8;        // 1 KB loads (8 rows) per step
+  constexpr int LPW = (NLD + NSUB - 1) / NSUB;
+  static_assert(NST >= 2 && (NST - 1) * LPW < 64, "stage count");
+  __shared__ __attribute__((aligned(16))) char smem[NST * STAGE];
   const GemmK& p = q.k;
   const int lane = threadIdx.x & 63;
   const int ns = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1325,49 +1335,68 @@ __global__ void __launch_bounds__(BNC * 2) gemm_f32_ksp_kernel(F32Ksp q) {
   map_tile(p.tiles_m, p.tiles_n, tmi, tni);
   const int g = blockIdx.y;
   const int64_t m0 = (int64_t)tmi * 32;
-  const int row = (int)min(m0 + (lane & 31), p.M - 1);  // rows past M re-read row M-1 (never stored)
-  const int h4 = 4 * (lane >> 5);
-  const int64_t k0 = g * q.kq, k1 = min(p.K, k0 + q.kq);
-  const int nsteps = k1 > k0 ? (int)((k1 - k0 + 7) / 8) : 0;
-  const char* Ab = (const char*)p.A;
-  const char* Bb = (const char*)p.B;
-  const uint32_t arow = (uint32_t)((int64_t)row * p.lda * 4);
-  const uint32_t brow = (uint32_t)(((int64_t)tni * BNC + ns * 32 + (lane & 31)) * p.ldb * 4);
-  const int64_t klast = k1 > k0 ? k1 - 4 : 0;
-  const uint32_t ring = (uint32_t)(uintptr_t)smem + (uint32_t)(ns * PD * STEP);
-  auto issue = [&](int st) {  // step st into ring slot st % PD (past the slice: the slice end again)
-    const int64_t k = k0 + 8 * (int64_t)st + h4;
-    const uint32_t kb = (uint32_t)(min(k, klast) * 4);
-    const uint32_t dst = ring + (uint32_t)((st % PD) * STEP);
-    dma_load16(Ab, arow + kb, dst);
-    dma_load16(Bb, brow + kb, dst + 1024);
+  const int hl = lane >> 5, h4 = 4 * hl;
+  const int k0 = (int)(g * q.kq), k1 = (int)min(p.K, g * q.kq + q.kq);
+  const int nsteps = k1 > k0 ? (k1 - k0 + 31) / 32 : 0;
+  const int klast = k1 > k0 ? k1 - 4 : 0;  // chunks past the slice re-read its last one, zeroed where used
+  // Load i of this wave is rows 8 (ns + i NSUB) .. + 8 of [lhs rows | packed rhs rows]
+  // (past the last row: that one again, the same bytes to the same place). Row R's
+  // 16-byte chunk c sits in slot c ^ (R & 7) ^ ((R >> 3) & 1).
+  uint32_t ro[LPW];
+  int kc[LPW];
+  const char* base[LPW];
+  uint32_t dst[LPW];
+#pragma unroll
+  for (int i = 0; i < LPW; ++i) {
+    const int grp = min(ns + i * NSUB, NLD - 1), r = 8 * grp + (lane >> 3);
+    kc[i] = 4 * ((lane & 7) ^ (lane >> 3) ^ (grp & 1));
+    const bool is_a = grp < 4;
+    base[i] = is_a ? (const char*)p.A : (const char*)p.B;
+    ro[i] = is_a ? (uint32_t)(min(m0 + r, p.M - 1) * p.lda * 4)  // rows past M re-read row M-1 (never stored)
+                 : (uint32_t)(((int64_t)tni * BNC + (r - 32)) * p.ldb * 4);
+    dst[i] = (uint32_t)(uintptr_t)smem + grp * 1024;
+  }
+  auto issue = [&](int st) {
+#pragma unroll
+    for (int i = 0; i < LPW; ++i)
+      dma_load16(base[i], ro[i] + (uint32_t)(min(k0 + 32 * st + kc[i], klast) * 4), dst[i] + (uint32_t)((st % NST) * STAGE));
   };
   f32x16_t acc;
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.f;
   float ss = 0.f;
-#pragma unroll
-  for (int j = 0; j < PD; ++j) issue(j);
+  const int sw = (lane & 7) ^ ((lane >> 3) & 1);
+  const int arow = (lane & 31) * 128, brow = (32 + ns * 32 + (lane & 31)) * 128;
+  const int pre = min(NST, nsteps);
+  for (int st = 0; st < pre; ++st) issue(st);
   for (int st = 0; st < nsteps; ++st) {
-    wait_vmcnt<2 * (PD - 1)>();  // step st landed; the PD - 1 later steps may be in flight
-    asm volatile("" ::: "memory");
-    const char* slotp = smem + ns * PD * STEP + (st % PD) * STEP;
-    float4 a = *(const float4*)(slotp + 16 * lane);
-    float4 b = *(const float4*)(slotp + 1024 + 16 * lane);
-    if (!(k0 + 8 * (int64_t)st + h4 < k1)) a = b = make_float4(0.f, 0.f, 0.f, 0.f);
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b.x, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b.y, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, b.z, acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b.w, acc, 0, 0, 0);
-    ss += a.x * a.x + a.y * a.y + a.z * a.z + a.w * a.w;  // (used only with sumsq)
-    asm volatile("" ::: "memory");
-    issue(st + PD);
-  }
-  wait_vmcnt<0>();  // no direct-to-LDS load lands after the workgroup ends
-  // partial subtile: rows 8(r/4) + 4(l/32) + r%4, column l%32 (32 lanes store 128 contiguous bytes)
-  float* dst = q.part + ((int64_t)g * q.Mp + m0 + h4) * q.Npk + (int64_t)tni * BNC + ns * 32 + (lane & 31);
+    // step st has landed everywhere; step st - 1's stage, read by every wave, is refilled
+    wait_tiles<LPW>(min(st == 0 ? NST - 1 : NST - 2, nsteps - 1 - st));
+    lds_barrier();
+    if (st > 0 && st - 1 + NST < nsteps) issue(st - 1 + NST);
+    const char* sp = smem + (st % NST) * STAGE;
+    float4 a[4], b[4];
 #pragma unroll
-  for (int r = 0; r < 16; ++r) dst[(int64_t)(8 * (r >> 2) + (r & 3)) * q.Npk] = acc[r];
+    for (int j = 0; j < 4; ++j) {
+      const int c = ((2 * j + hl) ^ sw) << 4;
+      a[j] = *(const float4*)(sp + arow + c);
+      b[j] = *(const float4*)(sp + brow + c);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (!(k0 + 32 * st + 8 * j + h4 < k1)) a[j] = b[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j].x, b[j].x, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j].y, b[j].y, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j].z, b[j].z, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j].w, b[j].w, acc, 0, 0, 0);
+      ss += a[j].x * a[j].x + a[j].y * a[j].y + a[j].z * a[j].z + a[j].w * a[j].w;  // (used only with sumsq)
+    }
+  }
+  // (every load issued was waited for: none lands after the workgroup ends)
+  // partial subtile: rows 8(r/4) + 4(l/32) + r%4, column l%32 (32 lanes store 128 contiguous bytes)
+  float* dp = q.part + ((int64_t)g * q.Mp + m0 + h4) * q.Npk + (int64_t)tni * BNC + ns * 32 + (lane & 31);
+#pragma unroll
+  for (int r = 0; r < 16; ++r) dp[(int64_t)(8 * (r >> 2) + (r & 3)) * q.Npk] = acc[r];
   if (p.sumsq && ns == 0 && tni == 0) {
     const float v = ss + __shfl_xor(ss, 32);
     if (lane < 32) q.ssq[(int64_t)g * q.Mp + m0 + lane] = v;
@@ -1428,7 +1457,7 @@ __global__ void __launch_bounds__(256) gemm_f32_ksr_kernel(F32Ksp q) {
 }
 
 // K slices of the split-K fp32 path for tiles 32-row x BNC tiles: about one
-// workgroup per CU, each slice at least two 8-wide steps. (Two per CU measured
+// workgroup per CU, each slice at least half a 32-wide step. (Two per CU measured
 // 15% slower on the fp32 block: twice the partial sums to write and re-read,
 // each workgroup's K slice little more than its load pipeline's depth.)
 static int f32_ksp_slices(int64_t tiles, int64_t K) {
@@ -1898,7 +1927,7 @@ extern "C" int th_gemm(const th_gemm_desc* d, void* stream) {
         q.Mp = (int64_t)k.tiles_m * 32;
         q.Npk = npk;
         q.ksg = f32_ksp_slices((int64_t)k.tiles_m * k.tiles_n, d->K);
-        q.kq = cdiv(cdiv(d->K, q.ksg), 8) * 8;
+        q.kq = cdiv(cdiv(d->K, q.ksg), 32) * 32;  // whole 128-byte lines
         q.ksg = (int)cdiv(d->K, q.kq);
         q.part = d->workspace;
         q.ssq = d->workspace + q.ksg * q.Mp * q.Npk;
