@@ -24,6 +24,14 @@
 //   last read, so a load has six phases (one and a half K steps) to land where
 //   a whole-stage double buffer gives it less than one.
 //   The next B0 lands in B1's registers: the two swap roles every K step.
+//   That holds only while the compiler adds no wait of its own to the loop: a load
+//   of the epilogue that may still be pending on some path, or a spilled register
+//   reloaded, makes it wait for every load in flight (tests/test_gemm_pp_schedule.py
+//   reads the assembly). So the epilogue loads nothing that it does not use, and the
+//   per-lane offsets are computed anew for each K loop instead of kept across the
+//   epilogue. (With such waits in 192-row tiles and spills in 256-row ones: fused RoPE
+//   16384 x 4096 x 4096 524 us, without 449; 16384 x 50280 x 1024 1756, without 1612;
+//   SwiGLU 3001 x 2 * 14336 x 4096 591, without 566.)
 // * K need only be a multiple of 8: the last two steps re-read columns, whose
 //   fragments are zeroed. (Two steps, so that the step count is even and every
 //   tile starts in stage 0 with B0 in the same registers; a branch on the
@@ -121,9 +129,9 @@ __device__ __forceinline__ void pp_epi(const GemmK& p, const EpiOutK& eo, int o2
 #pragma unroll
     for (int i = 0; i < NO; ++i) fetch(0, i);
   }
+  const int nt = (int)min((p.M - row_w + 31) >> 5, (int64_t)TM);  // (the caller has checked row_w < M)
 #pragma unroll 1
-  for (int t = 0; t < TM; ++t) {
-    if (row_w + 32 * t >= p.M) break;
+  for (int t = 0; t < nt; ++t) {
     // acc[t] to fixed registers, as octets
     float s[2][2][8];
 #define TH_PP_TAKE(T_)                                                                                        \
@@ -247,7 +255,7 @@ __device__ __forceinline__ void pp_epi(const GemmK& p, const EpiOutK& eo, int o2
       } else if constexpr (USES_E) {
         float xe[8];
         raw8_get(xr[i], p.extra_dtype[eo.e], xe);
-        if (t + 1 < TM) fetch(t + 1, i);  // this octet of the next row subtile
+        if (t + 1 < nt) fetch(t + 1, i);  // this octet of the next row subtile
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const float a = s[u][q][e];
@@ -317,8 +325,6 @@ __global__ void __launch_bounds__(512, 1) gemm_bf16_pp_kernel(GemmK p) {
 
   // LDS rows are 128 bytes (64 bf16), chunk c of row R in slot c ^ g(R), g(R) =
   // (R & 7) ^ ((R >> 3) & 1). Loads fill 8 rows (1 KB) each.
-  const int lrow = lane >> 3;
-  const uint32_t ch0 = (uint32_t)(((lane & 7) ^ lrow) << 4), ch1 = ch0 ^ 16u;
   // lhs: region A0 is rows wm' WM + 0 .. 32 T0 of both row halves, A1 the rest.
   // Wave w loads 4 T0 (4 T1) rows of row half w / 4 as T0 (T1) loads of 8 rows:
   // load i of region h is rows (w / 4) WM + 32 T0 h + 8 (i 4 + w % 4).
@@ -327,26 +333,31 @@ __global__ void __launch_bounds__(512, 1) gemm_bf16_pp_kernel(GemmK p) {
   // rhs: region B0 (B1) is subtile 0 (1) of the four N-waves, 128 rows; wave w
   // loads rows 16 (w % 2) .. + 16 of N-wave w / 2's subtile, as two loads of 8 rows.
   const int br0 = brow_of(wave >> 1, 0) + 16 * (wave & 1), br1 = brow_of(wave >> 1, 1) + 16 * (wave & 1);
-  const uint32_t vob0 = (uint32_t)(lrow * p.ldb * 2) + ch0;  // rows at an even multiple of 8
-  const uint32_t vob1 = (uint32_t)((8 + lrow) * p.ldb * 2) + ch1;
+  uint32_t vob0, vob1;
   const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
 
   const char *ga = nullptr, *gb0 = nullptr, *gb1 = nullptr;
-  auto tile_rsrc = [&](int L, int& tm, int& tn) {
-    pp_map(L, p.tiles_m, p.tiles_n, tm, tn);
-    const int64_t m0 = (int64_t)tm * BM;
-    const int arows = (int)min((int64_t)BM, p.M - m0);  // rows past M re-read row M - 1 (never stored)
-    ga = (const char*)p.A + m0 * p.lda * 2;
-    const char* gb = (const char*)p.B + (int64_t)tn * 256 * p.ldb * 2;
-    gb0 = gb + (int64_t)br0 * p.ldb * 2;
-    gb1 = gb + (int64_t)br1 * p.ldb * 2;
+  // Per-lane load offsets of tile row tm: set for the first loads of a tile, and again
+  // at the head of its K loop, so that the epilogue between the two need not keep them.
+  auto lane_offsets = [&](int tm) __attribute__((always_inline)) {
+    const int arows = (int)min((int64_t)BM, p.M - (int64_t)tm * BM);  // rows past M re-read row M - 1 (never stored)
     const int l = fresh_lane(), lr = l >> 3;
     const uint32_t c0 = (uint32_t)(((l & 7) ^ lr) << 4);
+    vob0 = (uint32_t)(lr * p.ldb * 2) + c0;  // rows at an even multiple of 8
+    vob1 = (uint32_t)((8 + lr) * p.ldb * 2) + (c0 ^ 16u);
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       const int r = i < T0 ? arow(0, i) : arow(1, i - T0);
       voa[i] = (uint32_t)(min(r + lr, arows - 1) * p.lda * 2) + ((r >> 3) & 1 ? c0 ^ 16u : c0);
     }
+  };
+  auto tile_rsrc = [&](int L, int& tm, int& tn) {
+    pp_map(L, p.tiles_m, p.tiles_n, tm, tn);
+    ga = (const char*)p.A + (int64_t)tm * BM * p.lda * 2;
+    const char* gb = (const char*)p.B + (int64_t)tn * 256 * p.ldb * 2;
+    gb0 = gb + (int64_t)br0 * p.ldb * 2;
+    gb1 = gb + (int64_t)br1 * p.ldb * 2;
+    lane_offsets(tm);
   };
   const int64_t k1 = (p.K - 8 * v2 - 64) * 2, k2 = (p.K - 64) * 2;
   auto kofs = [&](int kt) { return kt < nk - 2 ? (int64_t)kt * 128 : kt == nk - 2 ? k1 : k2; };
@@ -367,11 +378,15 @@ __global__ void __launch_bounds__(512, 1) gemm_bf16_pp_kernel(GemmK p) {
   using C1 = std::integral_constant<int, 1>;
 
   // fragment addresses: per 16-deep step ks, chunk 2 ks + lane / 32
-  int fch[4];
+  int fch[4], abase, bbase0, bbase1;
+  auto lane_fragments = [&]() __attribute__((always_inline)) {
+    const int l = fresh_lane();
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks) fch[ks] = ((ks * 2 + (lane >> 5)) ^ (lane & 7) ^ ((lane >> 3) & 1)) << 4;
-  const int abase = (wm * WM + (lane & 31)) * 128;
-  const int bbase0 = BBASE + (brow_of(wn, 0) + (lane & 31)) * 128, bbase1 = BBASE + (brow_of(wn, 1) + (lane & 31)) * 128;
+    for (int ks = 0; ks < 4; ++ks) fch[ks] = ((ks * 2 + (l >> 5)) ^ (l & 7) ^ ((l >> 3) & 1)) << 4;
+    abase = (wm * WM + (l & 31)) * 128;
+    bbase0 = BBASE + (brow_of(wn, 0) + (l & 31)) * 128;
+    bbase1 = BBASE + (brow_of(wn, 1) + (l & 31)) * 128;
+  };
 
   bf16x8_t fa[T0][4], fb[2][4];
   f32x16_t acc[TM][2];
@@ -563,6 +578,8 @@ __global__ void __launch_bounds__(512, 1) gemm_bf16_pp_kernel(GemmK p) {
     // B0(0) and A0(0) have landed everywhere, then the first B fragments
     wait_vmcnt<4 + TM + 2 + T1>();
     barrier_keep_loads();
+    lane_offsets(tmi);
+    lane_fragments();
     read_b(fb[0], bbase0, 0);
     ss[0] = ss[1] = ss[2] = ss[3] = 0.f;
 #pragma unroll
@@ -615,10 +632,11 @@ __global__ void __launch_bounds__(512, 1) gemm_bf16_pp_kernel(GemmK p) {
     const int gn0 = (int)col_t + c0 + 8 * ((le >> 5) + 2 * ((le >> 4) & 1));  // the lane's octet of a subtile
     const int lo = (int)col_t + c0, hi = lo + (NACC == 2 && !split ? 32 : jump + 32);
     const float* rsw = rsx + wm * WM;
-    for (int o = 0; o < pe.n_out; ++o) {
+    const int n_out = row_w < pe.M ? pe.n_out : 0;  // (a wave wholly past the last row has nothing to do)
+    for (int o = 0; o < n_out; ++o) {
       const EpiOutK& eo = pe.out[o];
       // an fp32 copy right after its bf16 output is stored from the same values
-      const int o2 = o + 1 < pe.n_out && same_values(eo, pe.out[o + 1]) ? o + 1 : -1;
+      const int o2 = o + 1 < n_out && same_values(eo, pe.out[o + 1]) ? o + 1 : -1;
       if (o2 >= 0) ++o;
       if (split && eo.a != (wn >> 1)) continue;
       if (eo.ce <= lo || eo.cb >= hi) continue;  // nothing of it in this wave
