@@ -55,3 +55,11 @@ def test_k_loop_keeps_loads_in_flight(kernels):
 def test_no_spills(kernels):
     for key, body in kernels.items():
         assert "scratch_" not in body, f"{key}: registers spill to scratch memory"
+
+
+def test_wide_buffer_stores_take_no_scalar_offset(kernels):
+    """The compiler keeps a wait between a 16-byte store and the next write of its data registers only for stores
+    without a register as scalar offset; with one, the last lanes' data was overwritten."""
+    for key, body in kernels.items():
+        stores = re.findall(r"buffer_store_dwordx4 v\[\d+:\d+\], v\d+, s\[\d+:\d+\], (\S+) ", body)
+        assert stores and set(stores) == {"0"}, key

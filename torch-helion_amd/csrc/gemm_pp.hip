@@ -75,60 +75,60 @@ __device__ __forceinline__ const GemmK& fresh_args() {
   return *(const GemmK*)a;
 }
 
-// Eight consecutive columns of one row, as loaded (bf16 in x, fp32 in x and y).
-struct Raw8 {
-  uint4 x, y;
-};
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ void raw8_load(Raw8& r, const void* p, int64_t off, int dtype) {
-  if (dtype == TH_BF16) {
-    r.x = *(const uint4*)((const uint16_t*)p + off);
-  } else {
-    r.x = *(const uint4*)((const float*)p + off);
-    r.y = *(const uint4*)((const float*)p + off + 4);
-  }
+// Buffer access to one wave's rows of an output or operand: the base is uniform, a lane's
+// offset 32 bits, and a lane with nothing to access has the offset kNone (or kNone and less than
+// 2 GiB more), which is past the end: its load is zero and its store dropped without a branch. (The compiler counts what is
+// in flight through straight-line code; around a branch it waits for everything.)
+constexpr uint32_t kNone = 0x80000000u;
+__device__ __forceinline__ auto wave_rows(const void* p, int64_t byte_off) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)((char*)p + byte_off), 0, 0x7fffffff, 0x00020000);
 }
 
-__device__ __forceinline__ void raw8_get(const Raw8& r, int dtype, float* v) {
-  const uint32_t w[8] = {r.x.x, r.x.y, r.x.z, r.x.w, r.y.x, r.y.y, r.y.z, r.y.w};
-  if (dtype == TH_BF16) {
+// acc[T] of this wave, lanes traded: afterwards octet s[u][q] of lane l is row 16 q + l % 16,
+// columns 8 (l / 32 + 2 (l / 16 % 2)) .. + 8 of column subtile u (NU of them).
+// Before, registers 8 q + j hold row l % 32, columns 16 q + 4 (l / 32) + j, and registers
+// 8 q + 4 + j the columns 8 further on. Swapping the upper half of registers 8 q + j with the
+// lower half of 8 q + 4 + j leaves columns 16 q + 8 (l / 32) + j and + 4 + j. Then q = 0 and 1
+// trade their odd and even rows of 16 lanes: q becomes the row half, and lane bits 5 and 4 are
+// column bits 3 and 4.
+template <int NU>
+__device__ __forceinline__ void trade_lanes(float (&s)[2][2][8]) {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      v[2 * q] = __uint_as_float(w[q] << 16);
-      v[2 * q + 1] = __uint_as_float(w[q] & 0xffff0000u);
+  for (int u = 0; u < NU; ++u) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const auto w = __builtin_amdgcn_permlane32_swap(__float_as_uint(s[u][q][j]), __float_as_uint(s[u][q][j + 4]),
+                                                        false, false);
+        s[u][q][j] = __uint_as_float(w[0]);
+        s[u][q][j + 4] = __uint_as_float(w[1]);
+      }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const auto w = __builtin_amdgcn_permlane16_swap(__float_as_uint(s[u][0][j]), __float_as_uint(s[u][1][j]),
+                                                      false, false);
+      s[u][0][j] = __uint_as_float(w[0]);
+      s[u][1][j] = __uint_as_float(w[1]);
     }
-  } else {
-#pragma unroll
-    for (int q = 0; q < 8; ++q) v[q] = __uint_as_float(w[q]);
   }
 }
 
-// One output op over the wave's TM row subtiles. Octet (u, q) of lane l is row
-// 16 q + l % 16 of a subtile, eight columns of column subtile u: accumulator
-// columns gn0 + u * jump .. + 8, gn0 the lane's own. TWO: the
+// One output op without further operands (ACC, SILU, SWIGLU) over the wave's TM row
+// subtiles: accumulator columns gn0 + u * jump .. + 8, gn0 the lane's own. TWO: the
 // column subtiles are the two accumulators' same columns (the op's own is eo.a).
 template <int OP, int TM, bool SUMSQ, bool TWO>
 __device__ __forceinline__ void pp_epi(const GemmK& p, const EpiOutK& eo, int o2, const f32x16_t (&acc)[TM][2],
                                        const float* rsw, int64_t row_w, int gn0, int jump, int lane) {
-  constexpr bool USES_E = OP == TH_EPI_ADD || OP == TH_EPI_SOFTPLUS_ADD || OP == TH_EPI_MUL;
-  constexpr bool USES_T = OP == TH_EPI_ROPE || OP == TH_EPI_ROPE_PAIR;
-  constexpr int NO = TWO ? 2 : 4;  // octets per row subtile
+  constexpr int NU = TWO ? 1 : 2;  // subtiles to store
   const bool sa = SUMSQ && ((p.rscale_mask >> eo.a) & 1u);
   const bool sb = SUMSQ && eo.b >= 0 && ((p.rscale_mask >> eo.b) & 1u);
   const int r_l = lane & 15;
-  auto gcol = [&](int i) { return gn0 + (TWO ? 0 : (i >> 1) * jump); };
+  auto gcol = [&](int u) { return gn0 + u * jump; };
   // (windows are multiples of 8, gemm_pp_fits: an octet is wholly in or out)
-  auto inside = [&](int i) { return gcol(i) >= eo.cb && gcol(i) < eo.ce; };
-  Raw8 xr[NO];
-  auto fetch = [&](int t, int i) __attribute__((always_inline)) {
-    const int64_t gm = row_w + 32 * t + 16 * (i & 1) + r_l;
-    if (inside(i) && gm < p.M)
-      raw8_load(xr[i], p.extra[eo.e], gm * p.ld_extra[eo.e] + gcol(i) - eo.cb, p.extra_dtype[eo.e]);
-  };
-  if constexpr (USES_E) {
-#pragma unroll
-    for (int i = 0; i < NO; ++i) fetch(0, i);
-  }
+  auto inside = [&](int u) { return gcol(u) >= eo.cb && gcol(u) < eo.ce; };
   const int nt = (int)min((p.M - row_w + 31) >> 5, (int64_t)TM);  // (the caller has checked row_w < M)
 #pragma unroll 1
   for (int t = 0; t < nt; ++t) {
@@ -139,10 +139,7 @@ __device__ __forceinline__ void pp_epi(const GemmK& p, const EpiOutK& eo, int o2
     if constexpr (T_ < TM) {                                                                                  \
       _Pragma("unroll") for (int u = 0; u < 2; ++u)                                                           \
           _Pragma("unroll") for (int q = 0; q < 2; ++q)                                                       \
-              _Pragma("unroll") for (int j = 0; j < 4; ++j) {                                                 \
-        s[u][q][j] = acc[T_ < TM ? T_ : 0][u][8 * q + j];                                                     \
-        s[u][q][j + 4] = acc[T_ < TM ? T_ : 0][u][8 * q + 4 + j];                                             \
-      }                                                                                                       \
+              _Pragma("unroll") for (int j = 0; j < 8; ++j) s[u][q][j] = acc[T_ < TM ? T_ : 0][u][8 * q + j]; \
     }                                                                                                         \
     break;
     switch (t) {
@@ -152,15 +149,14 @@ __device__ __forceinline__ void pp_epi(const GemmK& p, const EpiOutK& eo, int o2
       TH_PP_TAKE(3)
     }
 #undef TH_PP_TAKE
-    // Registers 8 q + j hold row l % 32, columns 16 q + 4 (l / 32) + j, registers
-    // 8 q + 4 + j the columns 8 further on. What needs no other operand is done here,
-    // so that it is done (and, for a bf16 output, rounded) before the lanes trade.
+    // The op is done here, so that it is done (and, for a bf16 output, rounded) before the
+    // lanes trade.
     const float rr = SUMSQ && (sa || sb) ? rsw[32 * t + (lane & 31)] : 1.f;
 #pragma unroll
     for (int q = 0; q < 2; ++q)
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        if constexpr (TWO) {  // own accumulator to s[0], the other one to s[1], by value
+        if constexpr (TWO) {  // own accumulator to s[0], by value
           const float x0 = s[0][q][e], x1 = s[1][q][e];
           float a = eo.a ? x1 : x0, bb = eo.b ? x1 : x0;
           if (sa) a *= rr;
@@ -168,7 +164,6 @@ __device__ __forceinline__ void pp_epi(const GemmK& p, const EpiOutK& eo, int o2
           if constexpr (OP == TH_EPI_SILU) a = a * sigmoidf_(a);
           if constexpr (OP == TH_EPI_SWIGLU) a = a * sigmoidf_(a) * bb;
           s[0][q][e] = a;
-          s[1][q][e] = bb;
         } else {
 #pragma unroll
           for (int u = 0; u < 2; ++u) {
@@ -179,13 +174,8 @@ __device__ __forceinline__ void pp_epi(const GemmK& p, const EpiOutK& eo, int o2
           }
         }
       }
-    // Swapping the upper half of registers 8 q + j with the lower half of 8 q + 4 + j
-    // leaves columns 16 q + 8 (l / 32) + j and + 4 + j. Then q = 0 and 1 trade their odd
-    // and even rows of 16 lanes: q becomes the row half, and lane bits 5 and 4 are
-    // column bits 3 and 4.
-    constexpr int NU = TWO && OP != TH_EPI_ROPE_PAIR ? 1 : 2;  // subtiles still needed
-    if (!USES_E && !USES_T && o2 < 0 && eo.dtype == TH_BF16) {
-      // packed pairs: half the exchanges
+    if (o2 < 0 && eo.dtype == TH_BF16) {
+      // packed pairs (trade_lanes on half the registers)
 #pragma unroll
       for (int u = 0; u < NU; ++u) {
         uint32_t w[2][4];
@@ -209,72 +199,186 @@ __device__ __forceinline__ void pp_epi(const GemmK& p, const EpiOutK& eo, int o2
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
           const int64_t gm = row_w + 32 * t + 16 * q + r_l;
-          if (gm < p.M && inside(2 * u + q))
-            *(uint4*)((uint16_t*)eo.ptr + gm * eo.ld + gcol(2 * u + q) - eo.cb) = make_uint4(w[q][0], w[q][1], w[q][2], w[q][3]);
+          if (gm < p.M && inside(u))
+            *(uint4*)((uint16_t*)eo.ptr + gm * eo.ld + gcol(u) - eo.cb) = make_uint4(w[q][0], w[q][1], w[q][2], w[q][3]);
         }
       }
       continue;
     }
+    trade_lanes<NU>(s);
 #pragma unroll
-    for (int u = 0; u < NU; ++u) {
+    for (int u = 0; u < NU; ++u)
 #pragma unroll
-      for (int q = 0; q < 2; ++q)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const auto w = __builtin_amdgcn_permlane32_swap(__float_as_uint(s[u][q][j]), __float_as_uint(s[u][q][j + 4]),
-                                                          false, false);
-          s[u][q][j] = __uint_as_float(w[0]);
-          s[u][q][j + 4] = __uint_as_float(w[1]);
+      for (int q = 0; q < 2; ++q) {
+        const int64_t gm = row_w + 32 * t + 16 * q + r_l;
+        if (gm < p.M && inside(u)) {
+          const int64_t gc = gcol(u) - eo.cb;
+          store8(eo.ptr, gm * eo.ld + gc, eo.dtype, true, 8, s[u][q]);
+          if (o2 >= 0) {
+            const EpiOutK& e2 = p.out[o2];
+            store8(e2.ptr, gm * e2.ld + gc, e2.dtype, true, 8, s[u][q]);
+          }
         }
+      }
+  }
+}
+
+// One output op with an operand per element over the wave's TM row subtiles, columns and
+// TWO as in pp_epi: KIND 0 the extra operand (ADD, SOFTPLUS_ADD, MUL; XB: it is bf16),
+// KIND 1 the RoPE tables (ROPE; TWO: ROPE_PAIR). What bounds it is the operand's latency:
+// the octets of the next subtile (of its next 16 rows, with four loads per octet for the
+// tables) are loaded before the present ones are stored, in code without branches around
+// memory accesses, so that the wait for them leaves the stores in flight. (Loaded octet by octet behind the stores instead, one serial round trip each:
+// residual with bf16 and fp32 outputs, 16384 x 1024 x 2048 @ADDP0@ us, now @ADDP1@; fused RoPE
+// 16384 x 4096 x 4096 @ROPE0@, now @ROPE1@.)
+template <int KIND, int TM, bool SUMSQ, bool TWO, bool XB, bool O2>
+__device__ __forceinline__ void pp_epi_x(const GemmK& p, const EpiOutK& eo, const EpiOutK& e2, const f32x16_t (&acc)[TM][2],
+                                         const float* rsw, int64_t row_w, int gn0, int jump, int lane) {
+  constexpr int NU = TWO ? 1 : 2;                    // subtiles to store
+  constexpr int NS = TWO && KIND == 0 ? 1 : 2;       // subtiles to trade
+  constexpr int ES = XB ? 2 : 4;                     // bytes of an operand element
+  constexpr int NX = KIND == 1 ? 4 : XB ? 1 : 2;     // 16-byte loads per octet
+  const bool sa = SUMSQ && ((p.rscale_mask >> eo.a) & 1u);
+  const bool sb = SUMSQ && eo.b >= 0 && ((p.rscale_mask >> eo.b) & 1u);
+  const int r_l = lane & 15;
+  const int rem = (int)min(p.M - row_w, (int64_t)32 * TM);  // rows of this wave
+  // byte offsets of the lane's octets in row r_l of the wave's rows
+  uint32_t vo[NU], v2[NU], vx[NU];
+  const int os = eo.dtype == TH_BF16 ? 2 : 4, os2 = e2.dtype == TH_BF16 ? 2 : 4;
+  const int ldx = KIND == 0 ? (int)p.ld_extra[eo.e] : 0;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const auto w = __builtin_amdgcn_permlane16_swap(__float_as_uint(s[u][0][j]), __float_as_uint(s[u][1][j]),
-                                                        false, false);
-        s[u][0][j] = __uint_as_float(w[0]);
-        s[u][1][j] = __uint_as_float(w[1]);
+  for (int u = 0; u < NU; ++u) {
+    const int gc = gn0 + u * jump;
+    const bool in = gc >= eo.cb && gc < eo.ce;  // (windows are multiples of 8: an octet is wholly in or out)
+    vo[u] = in ? (uint32_t)((r_l * (int)eo.ld + gc - eo.cb) * os) : kNone;
+    if constexpr (O2) v2[u] = in ? (uint32_t)((r_l * (int)e2.ld + gc - eo.cb) * os2) : kNone;
+    if constexpr (KIND == 0) vx[u] = in ? (uint32_t)((r_l * ldx + gc - eo.cb) * ES) : kNone;
+    else vx[u] = (uint32_t)(gc % p.hd) * 4;
+  }
+  const auto ro = wave_rows(eo.ptr, row_w * eo.ld * os);
+  const auto r2 = wave_rows(e2.ptr, O2 ? row_w * e2.ld * os2 : 0);
+  const auto rx = wave_rows(KIND == 0 ? p.extra[eo.e] : p.rcos, KIND == 0 ? row_w * ldx * ES : 0);
+  const auto rt = wave_rows(KIND == 0 ? p.extra[eo.e] : p.rsin, 0);
+  auto live = [&](uint32_t v, int row0) { return r_l < rem - row0 ? v : kNone; };
+
+  // RoPE: table row of the lane's rows, stepped by 16 (one division a tile)
+  uint32_t trow = 0;
+  const uint32_t period = (uint32_t)p.period, step16 = KIND == 1 ? 16u % period : 0u;
+  if constexpr (KIND == 1) trow = (uint32_t)(row_w + r_l) % period;
+  constexpr int NQ = KIND == 0 ? 2 : 1;  // row halves loaded at a time
+  u32x4_t x[NU][NQ][NX];
+  auto fetch = [&](int row0) __attribute__((always_inline)) {  // rows row0 .. + 16 NQ
+#pragma unroll
+    for (int q = 0; q < NQ; ++q)
+#pragma unroll
+      for (int u = 0; u < NU; ++u) {
+        if constexpr (KIND == 0) {
+          const uint32_t v = live(vx[u], row0 + 16 * q);
+          const int so = (row0 + 16 * q) * ldx * ES;
+#pragma unroll
+          for (int k = 0; k < NX; ++k) x[u][q][k] = __builtin_amdgcn_raw_buffer_load_b128(rx, v, so + 16 * k, 0);
+        } else {
+          const uint32_t v = trow * (uint32_t)p.hd * 4 + vx[u];
+#pragma unroll
+          for (int k = 0; k < 2; ++k) {
+            x[u][q][k] = __builtin_amdgcn_raw_buffer_load_b128(rx, v, 16 * k, 0);
+            x[u][q][2 + k] = __builtin_amdgcn_raw_buffer_load_b128(rt, v, 16 * k, 0);
+          }
+        }
+      }
+    if constexpr (KIND == 1) {
+      trow += step16;
+      trow = trow >= period ? trow - period : trow;
+    }
+  };
+  // (The offset goes in through the lane's register alone: with a scalar register as the store's
+  // own offset the compiler leaves out the wait between a 16-byte store and the next write of its
+  // data registers, and the last lanes' data was overwritten on this chip.)
+  auto put = [&](auto r, uint32_t v, int dtype, const float* f) __attribute__((always_inline)) {
+    if (dtype == TH_BF16) {
+      const u32x4_t w = {pk_bf16x2(f[0], f[1]), pk_bf16x2(f[2], f[3]), pk_bf16x2(f[4], f[5]), pk_bf16x2(f[6], f[7])};
+      __builtin_amdgcn_raw_buffer_store_b128(w, r, v, 0, 0);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const u32x4_t w = {__float_as_uint(f[4 * k]), __float_as_uint(f[4 * k + 1]), __float_as_uint(f[4 * k + 2]),
+                           __float_as_uint(f[4 * k + 3])};
+        __builtin_amdgcn_raw_buffer_store_b128(w, r, v + 16 * k, 0, 0);
       }
     }
+  };
+
+  fetch(0);
 #pragma unroll
-    for (int i = 0; i < NO; ++i) {
-      const int q = i & 1, u = i >> 1;
-      const int64_t gm = row_w + 32 * t + 16 * q + r_l;
-      float v[8];
-      if constexpr (USES_T) {
-        const int tcol = gcol(i) % p.hd;
-        const int64_t trow = (int64_t)((int)(gm % p.period)) * p.hd;
-        const float4 c0 = *(const float4*)(p.rcos + trow + tcol), c1 = *(const float4*)(p.rcos + trow + tcol + 4);
-        const float4 s0 = *(const float4*)(p.rsin + trow + tcol), s1 = *(const float4*)(p.rsin + trow + tcol + 4);
-        const float cs[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
-        const float sn[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+  for (int t = 0; t < TM; ++t) {  // (subtiles past M: nothing is loaded or stored)
+    float s[2][2][8];
+    const float rr = SUMSQ && (sa || sb) ? rsw[32 * t + (lane & 31)] : 1.f;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          // ROPE: the partner is the other subtile's same column
-          const float rot = TWO ? s[1][q][e] : u ? s[0][q][e] : -s[1][q][e];
-          v[e] = s[u][q][e] * cs[e] + rot * sn[e];
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float x0 = acc[t][0][8 * q + e], x1 = acc[t][1][8 * q + e];
+        float a = TWO && eo.a ? x1 : x0, b = TWO ? (eo.b ? x1 : x0) : x1;
+        if (sa) a *= rr;
+        if (TWO ? sb : sa) b *= rr;
+        s[0][q][e] = a;
+        s[1][q][e] = b;
+      }
+    trade_lanes<NS>(s);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int row0 = 32 * t + 16 * q;
+      if constexpr (KIND == 0) {
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+          float xe[8];
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            if constexpr (XB) {
+              xe[2 * k] = __uint_as_float(x[u][q][0][k] << 16);
+              xe[2 * k + 1] = __uint_as_float(x[u][q][0][k] & 0xffff0000u);
+            } else {
+              xe[k] = __uint_as_float(x[u][q][0][k]);
+              xe[4 + k] = __uint_as_float(x[u][q][NX - 1][k]);
+            }
+          }
+          float (&v)[8] = s[u][q];
+          if (eo.op == TH_EPI_MUL) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] *= xe[e];
+          } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] += xe[e];
+            if (eo.op == TH_EPI_SOFTPLUS_ADD) {
+#pragma unroll
+              for (int e = 0; e < 8; ++e) v[e] = softplusf_(v[e]);
+            }
+          }
         }
-      } else if constexpr (USES_E) {
-        float xe[8];
-        raw8_get(xr[i], p.extra_dtype[eo.e], xe);
-        if (t + 1 < nt) fetch(t + 1, i);  // this octet of the next row subtile
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float a = s[u][q][e];
-          if constexpr (OP == TH_EPI_MUL) v[e] = a * xe[e];
-          else if constexpr (OP == TH_EPI_ADD) v[e] = a + xe[e];
-          else v[e] = softplusf_(a + xe[e]);
-        }
+        if (q == 0) continue;  // (both halves were loaded together)
       } else {
+        // ROPE: the partner is the other subtile's same column. (The fma written out: left to
+        // contraction, which product it rounds could differ between two outputs of one value.)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = s[u][q][e];
-      }
-      if (gm < p.M && inside(i)) {
-        const int64_t gc = gcol(i) - eo.cb;
-        store8(eo.ptr, gm * eo.ld + gc, eo.dtype, true, 8, v);
-        if (o2 >= 0) {
-          const EpiOutK& e2 = p.out[o2];
-          store8(e2.ptr, gm * e2.ld + gc, e2.dtype, true, 8, v);
+        for (int e = 0; e < 8; ++e) {
+          const float a = s[0][q][e], b = s[1][q][e];
+          const int k = e >> 2, w = e & 3;
+          s[0][q][e] = fmaf(a, __uint_as_float(x[0][0][k][w]), (TWO ? b : -b) * __uint_as_float(x[0][0][2 + k][w]));
+          if constexpr (!TWO)
+            s[1][q][e] = fmaf(b, __uint_as_float(x[NU - 1][0][k][w]), a * __uint_as_float(x[NU - 1][0][2 + k][w]));
         }
       }
+      if (row0 + 16 < 32 * TM) fetch(row0 + 16);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int h = NQ == 2 ? 0 : q; h <= q; ++h)
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+          const int rs = 32 * t + 16 * h;
+          put(ro, live(vo[u] + rs * (int)eo.ld * os, rs), eo.dtype, s[u][h]);
+          if constexpr (O2) put(r2, live(v2[u] + rs * (int)e2.ld * os2, rs), e2.dtype, s[u][h]);
+        }
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
 }
@@ -443,7 +547,6 @@ __global__ void __launch_bounds__(512, 1) gemm_bf16_pp_kernel(GemmK p) {
         for (int ks = 0; ks < 4; ++ks) {
           // (a select of values, word by word: of array elements it would be one of
           // addresses, and the fragments would live in scratch memory)
-          typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
           const u32x4_t x0 = __builtin_bit_cast(u32x4_t, fa[0][ks]), x1 = __builtin_bit_cast(u32x4_t, fa[TH - 1][ks]);
           u32x4_t x = x0;
           if constexpr (TH > 1) {
@@ -640,29 +743,33 @@ __global__ void __launch_bounds__(512, 1) gemm_bf16_pp_kernel(GemmK p) {
       if (o2 >= 0) ++o;
       if (split && eo.a != (wn >> 1)) continue;
       if (eo.ce <= lo || eo.cb >= hi) continue;  // nothing of it in this wave
-#define TH_PP_CASE(OP_, TWO_)                                                            \
+#define TH_PP_CASE(OP_, TWO_)                                               \
   pp_epi<OP_, TM, SUMSQ, TWO_>(pe, eo, o2, acc, rsw, row_w, gn0, jump, le); \
   break
+#define TH_PP_X(KIND_, TWO_, XB_)                                                                          \
+  if (o2 >= 0)                                                                                             \
+    pp_epi_x<KIND_, TM, SUMSQ, TWO_, XB_, true>(pe, eo, pe.out[o2], acc, rsw, row_w, gn0, jump, le); \
+  else                                                                                                     \
+    pp_epi_x<KIND_, TM, SUMSQ, TWO_, XB_, false>(pe, eo, eo, acc, rsw, row_w, gn0, jump, le)
       if (NACC == 1 || split) {
         switch (eo.op) {
           case TH_EPI_ACC: TH_PP_CASE(TH_EPI_ACC, false);
-          case TH_EPI_ROPE: TH_PP_CASE(TH_EPI_ROPE, false);
           case TH_EPI_SILU: TH_PP_CASE(TH_EPI_SILU, false);
-          case TH_EPI_ADD: TH_PP_CASE(TH_EPI_ADD, false);
-          case TH_EPI_SOFTPLUS_ADD: TH_PP_CASE(TH_EPI_SOFTPLUS_ADD, false);
-          default: TH_PP_CASE(TH_EPI_MUL, false);
+          case TH_EPI_ROPE: TH_PP_X(1, false, false); break;
+          default:
+            if (pe.extra_dtype[eo.e] == TH_BF16) { TH_PP_X(0, false, true); } else { TH_PP_X(0, false, false); }
         }
       } else if constexpr (NACC == 2) {
         switch (eo.op) {
           case TH_EPI_ACC: TH_PP_CASE(TH_EPI_ACC, true);
-          case TH_EPI_ROPE_PAIR: TH_PP_CASE(TH_EPI_ROPE_PAIR, true);
           case TH_EPI_SILU: TH_PP_CASE(TH_EPI_SILU, true);
           case TH_EPI_SWIGLU: TH_PP_CASE(TH_EPI_SWIGLU, true);
-          case TH_EPI_ADD: TH_PP_CASE(TH_EPI_ADD, true);
-          case TH_EPI_SOFTPLUS_ADD: TH_PP_CASE(TH_EPI_SOFTPLUS_ADD, true);
-          default: TH_PP_CASE(TH_EPI_MUL, true);
+          case TH_EPI_ROPE_PAIR: TH_PP_X(1, true, false); break;
+          default:
+            if (pe.extra_dtype[eo.e] == TH_BF16) { TH_PP_X(0, true, true); } else { TH_PP_X(0, true, false); }
         }
       }
+#undef TH_PP_X
 #undef TH_PP_CASE
     }
     if (!more) break;
@@ -677,15 +784,18 @@ __global__ void __launch_bounds__(512, 1) gemm_bf16_pp_kernel(GemmK p) {
 // Operand and output forms the kernel covers (th_gemm has checked the rest).
 bool gemm_pp_fits(const GemmK& k) {
   if (k.K < 128 || k.M >= ((int64_t)1 << 31) || k.N >= ((int64_t)1 << 31)) return false;
-  if ((int64_t)256 * k.lda * 2 >= ((int64_t)1 << 31) || (int64_t)256 * k.ldb * 2 >= ((int64_t)1 << 31)) return false;
+  constexpr int64_t two_gib = (int64_t)1 << 31;
+  auto rows_fit = [](int64_t ld, int bytes) { return ld < two_gib / (256 * bytes); };
+  if (!rows_fit(k.lda, 2) || !rows_fit(k.ldb, 2)) return false;
   if (!((k.n_acc == 1 && k.bn == 256) || (k.n_acc == 2 && k.bn == 128))) return false;
   bool rope = false, pair = false;
   for (int o = 0; o < k.n_out; ++o) {
     rope |= k.out[o].op == TH_EPI_ROPE;
     pair |= k.out[o].b >= 0;
-    // whole aligned octets in every output and operand row
-    if (!k.out[o].vec8 || k.out[o].ce % 8 != 0) return false;
-    if (k.out[o].e >= 0 && !k.extra_vec8[k.out[o].e]) return false;
+    // whole aligned octets in every output and operand row, a tile's rows within 2 GiB
+    if (!k.out[o].vec8 || k.out[o].ce % 8 != 0 || !rows_fit(k.out[o].ld, 4)) return false;
+    if (k.out[o].e >= 0 && (!k.extra_vec8[k.out[o].e] || !rows_fit(k.ld_extra[k.out[o].e], 4))) return false;
+    if ((k.out[o].op == TH_EPI_ROPE || k.out[o].op == TH_EPI_ROPE_PAIR) && (int64_t)k.period * k.hd * 4 >= two_gib) return false;
   }
   // fused RoPE: heads of 64 and wider, whose partners meet in a wave (narrower
   // ones would need columns of other lanes); two accumulators: whole-accumulator
