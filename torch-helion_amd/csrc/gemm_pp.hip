@@ -500,7 +500,7 @@ __global__ void __launch_bounds__(512, 1) gemm_bf16_pp_kernel(GemmK p) {
   // tiles walk down the columns of eight tile rows, mostly along one row, and
   // the scales stay in LDS.
   float ss[4];
-  bool need_ss = SUMSQ;
+  bool new_row = SUMSQ, need_ss = SUMSQ && p.rs_parts == nullptr;
   const bf16x8_t zero8 = {};
   auto read_a = [&](auto hc, int st) __attribute__((always_inline)) {
     constexpr int H = decltype(hc)::value;
@@ -674,6 +674,13 @@ __global__ void __launch_bounds__(512, 1) gemm_bf16_pp_kernel(GemmK p) {
   int L = blockIdx.x;
   if (L >= tiles) return;
   int tmi, tni;
+  // scale of the tile row's row r, whose own sum of squares is `own` (unless the producer's parts are given)
+  auto row_scale = [&](int r, float own) __attribute__((always_inline)) {
+    const int64_t gr = (int64_t)tmi * BM + r;
+    const float v = row_sumsq(p, gr, own);
+    rsx[r] = rsqrtf(v * p.inv_k + p.eps);
+    if (p.sumsq_out && gr < p.M) p.sumsq_out[gr] = v;  // (every workgroup of the row writes the same value)
+  };
   tile_rsrc(L, tmi, tni);
   start_tile();
 
@@ -691,6 +698,15 @@ __global__ void __launch_bounds__(512, 1) gemm_bf16_pp_kernel(GemmK p) {
       for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[t][u][r] = 0.f;
+    if constexpr (SUMSQ) {
+      // Row scales from the producer's partial sums: here, where the tile's first loads are in
+      // flight (after the K loop nothing is, and every wave waits), and past the barrier behind
+      // which no wave reads the last tile row's scales.
+      if (new_row && p.rs_parts != nullptr && wn < TM) {
+        const int r = fresh_lane();
+        if (r < 32) row_scale(wm * WM + 32 * wn + r, 0.f);
+      }
+    }
     mem_end();
     if (wm) mfma_end();  // the half-phase offset of the second group
 
@@ -705,14 +721,8 @@ __global__ void __launch_bounds__(512, 1) gemm_bf16_pp_kernel(GemmK p) {
     kstep(nk - 1, C1{}, M2{});
     if constexpr (SUMSQ) {
       const float own = (ss[0] + ss[1]) + (ss[2] + ss[3]);
-      float v = own + __shfl_xor(own, 32);
-      if (need_ss && wn < TM && lane < 32) {
-        const int r = wm * WM + 32 * wn + lane;
-        const int64_t gr = (int64_t)tmi * BM + r;
-        v = row_sumsq(p, gr, v);
-        rsx[r] = rsqrtf(v * p.inv_k + p.eps);
-        if (p.sumsq_out && gr < p.M) p.sumsq_out[gr] = v;  // (every workgroup of the row writes the same value)
-      }
+      const float v = own + __shfl_xor(own, 32);
+      if (need_ss && wn < TM && lane < 32) row_scale(wm * WM + 32 * wn + lane, v);
     }
     wait_lgkmcnt0();
     mfma_end();
@@ -774,7 +784,8 @@ __global__ void __launch_bounds__(512, 1) gemm_bf16_pp_kernel(GemmK p) {
     }
     if (!more) break;
     L = Ln;
-    need_ss = SUMSQ && tmn != tmi;
+    new_row = SUMSQ && tmn != tmi;
+    need_ss = new_row && p.rs_parts == nullptr;
     tmi = tmn;
     tni = tnn;
   }
