@@ -27,9 +27,9 @@
 //   That holds only while the compiler adds no wait of its own to the loop: a load
 //   of the epilogue that may still be pending on some path, or a spilled register
 //   reloaded, makes it wait for every load in flight (tests/test_gemm_pp_schedule.py
-//   reads the assembly). So the epilogue loads nothing that it does not use, and the
-//   per-lane offsets are computed anew for each K loop instead of kept across the
-//   epilogue. (With such waits in 192-row tiles and spills in 256-row ones: fused RoPE
+//   reads the assembly). So the epilogue loads nothing that it does not use, and with
+//   256 rows the per-lane offsets are computed anew for each K loop instead of kept
+//   across the epilogue. (With such waits in 192-row tiles and spills in 256-row ones: fused RoPE
 //   16384 x 4096 x 4096 524 us, without 449; 16384 x 50280 x 1024 1756, without 1612;
 //   SwiGLU 3001 x 2 * 14336 x 4096 591, without 566.)
 // * K need only be a multiple of 8: the last two steps re-read columns, whose
@@ -442,8 +442,8 @@ __global__ void __launch_bounds__(512, 1) gemm_bf16_pp_kernel(GemmK p) {
   const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
 
   const char *ga = nullptr, *gb0 = nullptr, *gb1 = nullptr;
-  // Per-lane load offsets of tile row tm: set for the first loads of a tile, and again
-  // at the head of its K loop, so that the epilogue between the two need not keep them.
+  // Per-lane load offsets of tile row tm: set for the first loads of a tile, and with 256
+  // rows again at the head of its K loop, so that the epilogue between need not keep them.
   auto lane_offsets = [&](int tm) __attribute__((always_inline)) {
     const int arows = (int)min((int64_t)BM, p.M - (int64_t)tm * BM);  // rows past M re-read row M - 1 (never stored)
     const int l = fresh_lane(), lr = l >> 3;
@@ -684,13 +684,23 @@ __global__ void __launch_bounds__(512, 1) gemm_bf16_pp_kernel(GemmK p) {
   };
   tile_rsrc(L, tmi, tni);
   start_tile();
+  if constexpr (TM < 4) lane_fragments();
 
   for (;;) {
+    if constexpr (TM == 4) {
+      // (pinned here, where the tile's first loads are in flight: the compiler would compute the
+      // offsets past the barrier, 0.3 us of a tile)
+      lane_offsets(tmi);
+      lane_fragments();
+      asm volatile("" : "+v"(vob0), "+v"(vob1), "+v"(abase), "+v"(bbase0), "+v"(bbase1));
+#pragma unroll
+      for (int i = 0; i < TM; ++i) asm volatile("" : "+v"(voa[i]));
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) asm volatile("" : "+v"(fch[ks]));
+    }
     // B0(0) and A0(0) have landed everywhere, then the first B fragments
     wait_vmcnt<4 + TM + 2 + T1>();
     barrier_keep_loads();
-    lane_offsets(tmi);
-    lane_fragments();
     read_b(fb[0], bbase0, 0);
     ss[0] = ss[1] = ss[2] = ss[3] = 0.f;
 #pragma unroll
