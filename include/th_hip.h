@@ -182,6 +182,25 @@ int64_t th_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t n_acc, 
 /* One OpIR gemm KernelSpec. */
 int th_gemm(const th_gemm_desc* desc, void* stream);
 
+/* Main loops of th_gemm. */
+typedef enum th_gemm_loop {
+  TH_LOOP_FP8 = 0,         /* e4m3 weights */
+  TH_LOOP_F32 = 1,
+  TH_LOOP_F32_SPLIT = 2,   /* K split over workgroups, through the workspace */
+  TH_LOOP_F32_WAVES = 3,   /* K split over a workgroup's waves */
+  TH_LOOP_BF16_STAGED = 4,
+  TH_LOOP_BF16_DIRECT = 5,
+  TH_LOOP_BF16_PERSISTENT = 6,
+  TH_LOOP_BF16_PINGPONG = 7
+} th_gemm_loop;
+
+/* What th_gemm would run for this descriptor: route[0] = th_gemm_loop, route[1]
+ * and route[2] = rows and packed columns of a workgroup's tile; *us = the time
+ * that a bf16 loop is estimated to take on the device, without its launch (0 for
+ * the other types). Launches nothing and reads no operand (their pointers count
+ * only for alignment); without an initialised device, for 256 compute units. */
+int th_gemm_route(const th_gemm_desc* desc, int32_t* route, double* us);
+
 /* th_gemm that allocates nothing and takes no workspace. No counterpart in the
  * reference: it is for callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops such as the decode step, harnesses

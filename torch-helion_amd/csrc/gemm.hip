@@ -1557,16 +1557,34 @@ static int choose_bn(int64_t N, int n_acc, int in_dtype) {
   }
 }
 
-// About what the direct loop takes (us) on `tiles` 64-row tiles bnc columns wide and
-// nk 64-deep K steps, to compare with gemm_pp_rows's estimate. Measured: 64 x 256 tiles
-// 0.66 us per step whether 16 or 176 of them run (M = 128 .. 700, N = 4096, K = 512 ..
-// 4096), 0.8 - 0.9 on all 256 CUs, 64 x 128 tiles 0.43; two workgroups on a CU, up to
-// twice as many tiles, 1.3 and 0.58; narrower tiles are taken as the 128-wide ones.
-static double dl64_us(int64_t tiles, int64_t nk, int bnc, int64_t cus) {
-  const double per1 = bnc > 128 ? 0.66 : 0.43, per2 = bnc > 128 ? 1.3 : 0.58;
-  const double crowd = bnc > 128 ? std::max(0.0, (double)tiles / (double)cus - 0.7) * 0.7 : 0.0;
-  if (tiles <= cus) return 6 + nk * (per1 + crowd);
-  return 6 + (double)cdiv(tiles, 2 * cus) * nk * per2;
+// About what the 64-row direct loop and the 128- and 256-row persistent loops take (us) on
+// bm-row tiles bnc columns wide, to compare with gemm_pp_rows's estimate (fitted with it).
+// The direct loop: 64 x 256 tiles 0.76 us per 64-deep step, more where nearly all 256 CUs
+// have one, narrower tiles 0.42; two workgroups on a CU, up to twice as many tiles, 1.13 and
+// 0.56. The persistent loops by rounds; their epilogue is the cheaper one where the K loop is
+// short (16384 x 2048 x 192: 29.5 us against 33.5; x 320 36.1 against 41.5; x 576 48.5 against
+// 51.9), the dearer one for column windows and ragged rows (16384 x 2192 x 512 in five windows:
+// 86.2 against 68.0) and residuals (2067 x 20352 x 256: 74 against 54). One round of 128 x 128 tiles beats half a round of 128 x 256 ones
+// (4096 x 1024 x 1024 rotated: 19.3 us, and 18.4 on 64-row tiles, against 24.9).
+static double bf16_loop_us(const GemmK& k, const EpiCost& ec, int bm, int bnc, int64_t cus) {
+  const int64_t tiles = cdiv(k.M, bm) * k.tiles_n;
+  const double nk = (double)cdiv(k.K, 64), outs = ec.outs - 1;
+  const bool full = bnc > 128;  // 256 packed columns
+  if (bm == 64) {
+    const double load = (double)tiles / (double)cus;
+    const double t = 4.4 + 1.3 * load + ec.wide * (1.53 + 0.941 * load) + 1.08 * outs +
+                     (k.sumsq && k.rs_parts == nullptr ? 1.93 : 0);
+    if (tiles > cus) return t + 0.384 + (double)cdiv(tiles, 2 * cus) * nk * (full ? 1.13 : 0.557);
+    return t + nk * (full ? 0.756 + 0.512 * std::max(0.0, load - 0.7) : 0.419);
+  }
+  const int64_t rounds = cdiv(tiles, cus);
+  const double fill = (double)tiles / (double)(rounds * cus);
+  const double busy = fill * std::min(1.0, (double)rounds * nk / 256);
+  if (bm == 256)
+    return (double)rounds * (nk * (1.12 + 0.413 * fill + 0.172 * busy) + 10.5 + 4.61 * ec.rope + 0.857 * outs +
+                             fill * (std::max(ec.extra ? 6.0 : 0.0, 4.62 * ec.wide) + (ec.ragged ? 1.53 : 0)));
+  const double loop = full ? nk * (0.692 + 0.261 * fill) + 8.14 : std::max(7.59, 0.892 * nk);
+  return (double)rounds * (loop + 0.0247 * nk * busy + 4.41 * ec.wide + 5.9 * ec.rope + 1.26 * outs);
 }
 
 static int64_t packed_kp(int64_t K, int in_dtype) {
@@ -1766,7 +1784,16 @@ static void launch_f32_ksp(const F32Ksp& q, hipStream_t s) {
     hipLaunchKernelGGL((gemm_f32_ksr_kernel<BNC, 8>), dim3((unsigned)(q.Mp / 8 * q.k.tiles_n)), dim3(256), 0, s, q);
 }
 
-extern "C" int th_gemm(const th_gemm_desc* d, void* stream) {
+// th_gemm, or with `route` only what it would run: main loop, tile rows and columns, and in
+// *us the estimate that a bf16 loop was chosen by.
+static int gemm_run(const th_gemm_desc* d, void* stream, int32_t* route, double* us) {
+  auto only_route = [&](int loop, int64_t rows, int64_t cols) {
+    if (route == nullptr) return false;
+    route[0] = loop;
+    route[1] = (int32_t)rows;
+    route[2] = (int32_t)cols;
+    return true;
+  };
   TH_CHECK_ARG(d != nullptr, "th_gemm: null descriptor");
   TH_CHECK_ARG(d->M > 0 && d->N > 0 && d->K > 0, "th_gemm: M=%lld N=%lld K=%lld must be positive",
                (long long)d->M, (long long)d->N, (long long)d->K);
@@ -1899,7 +1926,7 @@ extern "C" int th_gemm(const th_gemm_desc* d, void* stream) {
   k.ss_parts_out = d->ss_parts_out;
   k.ld_ss_parts_out = d->ld_ss_parts_out;
   k.gain_index = d->gain_out_index;
-  if (!device_ready()) {
+  if (route == nullptr && !device_ready()) {
     set_error("th_gemm: th_init was not called for the current device");
     return TH_ERR_NOT_INIT;
   }
@@ -1909,6 +1936,7 @@ extern "C" int th_gemm(const th_gemm_desc* d, void* stream) {
   k.tiles_n = (int)cdiv(d->N, bn);
   if (fp8) {
     k.tiles_m = 1;
+    if (only_route(TH_LOOP_FP8, d->M, bnc)) return TH_OK;
     return launch_gemm_fp8(k, cdiv(d->N, bn) * bnc, d->rhs_scale, d->workspace, d->workspace_bytes, s);
   }
   if (d->in_dtype == TH_F32) {
@@ -1922,6 +1950,7 @@ extern "C" int th_gemm(const th_gemm_desc* d, void* stream) {
       if (d->workspace && d->workspace_bytes >= f32_ksp_bytes(d->M, npk, d->K, bnc) &&
           ((uintptr_t)d->workspace & 15) == 0) {
         // too few 64-row tiles to occupy the GPU: K split over workgroups through the workspace
+        if (only_route(TH_LOOP_F32_SPLIT, 32, bnc)) return TH_OK;
         F32Ksp q{};
         q.k = k;
         q.Mp = (int64_t)k.tiles_m * 32;
@@ -1942,6 +1971,7 @@ extern "C" int th_gemm(const th_gemm_desc* d, void* stream) {
         return TH_OK;
       }
       // without a workspace: 32-row tiles with the K loop split over the waves of a workgroup
+      if (only_route(TH_LOOP_F32_WAVES, 32, bnc)) return TH_OK;
       switch (bnc) {
         case 64: launch_f32_sk<64>(k, s); break;
         case 128: launch_f32_sk<128>(k, s); break;
@@ -1952,6 +1982,7 @@ extern "C" int th_gemm(const th_gemm_desc* d, void* stream) {
       TH_CHECK_LAUNCH();
       return TH_OK;
     }
+    if (only_route(TH_LOOP_F32, 64, bnc)) return TH_OK;
     k.tiles_m = (int)cdiv(d->M, 64);
     switch (bnc) {
       case 64: launch_f32<64>(k, s); break;
@@ -1991,19 +2022,26 @@ extern "C" int th_gemm(const th_gemm_desc* d, void* stream) {
       set_error("th_gemm: rs_parts is not implemented with whole-head RoPE on two accumulators");
       return TH_ERR_UNSUPPORTED;
     }
-    // The ping-pong kernel on 256-column tiles, where it is the faster one. (Narrower
-    // packed tiles of one accumulator are its columns in order, padded to the tile, so
-    // a multiple of 256 columns reads as 256-wide tiles too.)
+    // The ping-pong kernel on 256-column tiles, where it is estimated the faster one, or the
+    // loop it is compared with is not there (partial K steps; heads wider than a wave's columns
+    // on the larger tiles). (Narrower packed tiles of one accumulator are its columns in order,
+    // padded to the tile, so a multiple of 256 columns reads as 256-wide tiles too.)
     GemmK kp = k;
     if (d->n_acc == 1 && bn == 128 && d->N % 256 == 0) {
       kp.bn = 256;
       kp.tiles_n = (int)(d->N / 256);
     }
+    const EpiCost ec = gemm_epi_cost(k);
+    const double t_loop = bf16_loop_us(k, ec, bm, bnc, cus);
+    if (us != nullptr) *us = t_loop;
     if (gemm_pp_fits(kp)) {
       double t_pp = 0;
-      const int pbm = gemm_pp_rows(kp, cus, &t_pp);
-      if (!direct || bm > 64 || t_pp < dl64_us(k.tiles_m * (int64_t)k.tiles_n, d->K / 64, bnc, cus))
+      const int pbm = gemm_pp_rows(kp, ec, cus, &t_pp);
+      if (!direct || (bm > 64 && !wave_epi) || t_pp < t_loop) {
+        if (us != nullptr) *us = t_pp;
+        if (only_route(TH_LOOP_BF16_PINGPONG, pbm, 256)) return TH_OK;
         return launch_gemm_pp(kp, pbm, s);
+      }
     }
     MainLoop ml = MainLoop::staged;
     if (direct) ml = wave_epi ? MainLoop::persistent : MainLoop::direct;
@@ -2012,6 +2050,9 @@ extern "C" int th_gemm(const th_gemm_desc* d, void* stream) {
       k.tiles_m = (int)cdiv(d->M, 128);
       bm = 128;
     }
+    if (only_route(ml == MainLoop::persistent ? TH_LOOP_BF16_PERSISTENT
+                   : ml == MainLoop::direct ? TH_LOOP_BF16_DIRECT : TH_LOOP_BF16_STAGED, bm, bnc))
+      return TH_OK;
     switch (bnc) {
       case 64: bm == 64 ? launch_bf16_any<64, 64>(k, ml, s) : big ? launch_bf16_any<256, 64>(k, ml, s) : launch_bf16_any<128, 64>(k, ml, s); break;
       case 128: bm == 64 ? launch_bf16_any<64, 128>(k, ml, s) : big ? launch_bf16_any<256, 128>(k, ml, s) : launch_bf16_any<128, 128>(k, ml, s); break;
@@ -2022,4 +2063,12 @@ extern "C" int th_gemm(const th_gemm_desc* d, void* stream) {
   }
   TH_CHECK_LAUNCH();
   return TH_OK;
+}
+
+extern "C" int th_gemm(const th_gemm_desc* d, void* stream) { return gemm_run(d, stream, nullptr, nullptr); }
+
+extern "C" int th_gemm_route(const th_gemm_desc* d, int32_t* route, double* us) {
+  TH_CHECK_ARG(route != nullptr && us != nullptr, "th_gemm_route: null route or us");
+  *us = 0;
+  return gemm_run(d, nullptr, route, us);
 }

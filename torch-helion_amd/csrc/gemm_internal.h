@@ -198,7 +198,7 @@ __device__ __forceinline__ void store8(void* p, int64_t off, int dtype, bool vec
 
 // Outputs o and o + 1 compute the same values (same op, operands and column
 // window; only the destination differs).
-__device__ __forceinline__ bool same_values(const EpiOutK& x, const EpiOutK& y) {
+__host__ __device__ __forceinline__ bool same_values(const EpiOutK& x, const EpiOutK& y) {
   return x.op == y.op && x.a == y.a && x.b == y.b && x.e == y.e && x.cb == y.cb && x.ce == y.ce;
 }
 
@@ -212,9 +212,39 @@ __device__ __forceinline__ float sumsq8_dot(bf16x8_t v, float acc) {
   return acc;
 }
 
+// What a GEMM's epilogue adds to the time of a tile, in the terms of the estimates that
+// choose a main loop. An output that repeats the one before it (an fp32 copy) counts for
+// nothing, so that a value's bits do not depend on whether a copy is stored beside it.
+struct EpiCost {
+  double rope;  // share of the columns that are rotated
+  double wide;  // bytes stored and loaded per column beyond the 4 that every loop hides
+  bool ragged;  // output rows that are not whole 128-byte lines
+  bool extra;   // an operand per element
+  int outs;
+};
+
+inline EpiCost gemm_epi_cost(const GemmK& k) {
+  EpiCost c{0, 0, false, false, 0};
+  double bytes = 0;
+  const double cols = (double)k.N * k.n_acc;
+  for (int o = 0; o < k.n_out; ++o) {
+    const EpiOutK& eo = k.out[o];
+    if (o > 0 && same_values(k.out[o - 1], eo)) continue;
+    const double w = (double)(eo.ce - eo.cb) / cols;
+    bytes += 2 * w;
+    if (eo.e >= 0) bytes += w * (k.extra_dtype[eo.e] == TH_F32 ? 4 : 2);
+    if (eo.op == TH_EPI_ROPE || eo.op == TH_EPI_ROPE_PAIR) c.rope += w;
+    c.ragged |= eo.ld % 64 != 0 && eo.op != TH_EPI_SWIGLU;  // (SwiGLU is stored from registers in every loop)
+    c.extra |= eo.e >= 0;
+    ++c.outs;
+  }
+  c.wide = bytes > 4 ? bytes - 4 : 0;
+  return c;
+}
+
 // ping-pong persistent bf16 kernel (gemm_pp.hip)
 bool gemm_pp_fits(const GemmK& k);
-int gemm_pp_rows(const GemmK& k, int64_t cus, double* us);
+int gemm_pp_rows(const GemmK& k, const EpiCost& ec, int64_t cus, double* us);
 int launch_gemm_pp(const GemmK& k, int bm, hipStream_t s);
 
 int64_t fp8_workspace_bytes(int64_t M, int64_t Npk, int64_t K, int bn, int n_acc);

@@ -48,6 +48,8 @@
 //   (32 bytes per row, without the second swap, made a SwiGLU tile's stores 14%
 //   of a K = 1024 launch slower), and the next tile's first two K steps load
 //   under it.
+#include <algorithm>
+
 #include "gemm_internal.h"
 
 namespace th {
@@ -350,7 +352,9 @@ __device__ __forceinline__ void pp_epi_x(const GemmK& p, const EpiOutK& eo, cons
           } else {
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] += xe[e];
-            if (eo.op == TH_EPI_SOFTPLUS_ADD) {
+            // (a branch on the wave, not around memory accesses: a Mamba block's dt window is 16
+            // columns of a tile, and 64 lanes' softplus of the subtile beside it cost 1 us)
+            if (eo.op == TH_EPI_SOFTPLUS_ADD && __any(vo[u] != kNone)) {
 #pragma unroll
               for (int e = 0; e < 8; ++e) v[e] = softplusf_(v[e]);
             }
@@ -828,22 +832,29 @@ bool gemm_pp_fits(const GemmK& k) {
 }
 
 // Rows of the tile: the choice of 256, 192 and 128 with the smallest estimate (us, in
-// *us) of rounds * (K steps * per-step time + per-tile time). A step's time grows with
-// the share of the CUs at work (the clock falls: 256-row steps measured 0.94 us on 4
-// CUs, 1.25 on 192, 1.45 - 1.6 on all 256; 192-row steps 0.75, 0.82 at half, 1.2;
-// 128-row steps 0.47, 0.68 at three quarters, 0.75 - 0.93). Measured choices (us,
-// 256 / 192 / 128 rows): 3001 x 4096 x 14336 284 / 276 / 317; 16384 x 4096 x 14336
-// 1447 / 1756 / 1673; 2000 x 2 x 5632 x 2048 98 / 93 / 94; 1500 x 2048 x 4096 73 / 65 / 43.
-int gemm_pp_rows(const GemmK& k, int64_t cus, double* us) {
+// *us) of rounds * (K steps * per-step time + per-tile time), the K steps an even number.
+// A step's time grows with the share of the CUs at work, and by another 0.1 us once they are
+// at work for long (the clock falls: 256-row steps measured 0.94 us on 4 CUs, 1.25 on 192,
+// 1.45 - 1.6 on all 256; 192-row steps 0.75, 0.82 at half, 1.1 - 1.2; 128-row steps 0.47, 0.68
+// at three quarters, 0.75 - 0.93). Own sums of squares cost 0.14 us a step where a
+// workgroup's tile row is new, rotated tiles 6 us, a residual in fp32 2 to 10 us.
+// The constants here and in bf16_loop_us (gemm.hip) are fitted to what the choice among the
+// loops loses over 2125 shapes, each loop timed on each (32 .. 16384 rows, K = 128 .. 14336,
+// N = 256 .. 50280, eight kinds of outputs, sizes drawn as well as round): 0.4% of the time
+// on average; 0.7% over 467 drawn shapes that the fit has not seen.
+int gemm_pp_rows(const GemmK& k, const EpiCost& ec, int64_t cus, double* us) {
   static const struct { int bm; double c0, c1, e; } shape[] = {
-      {256, 0.85, 0.60, 13}, {192, 0.65, 0.50, 10}, {128, 0.45, 0.35, 8}};
-  const double nk = (double)cdiv(k.K, 64);
+      {256, 0.868, 0.570, 12.0}, {192, 0.611, 0.454, 9.91}, {128, 0.465, 0.243, 8.14}};
+  const double nk = 2.0 * (double)cdiv(k.K, 128);
+  const double own_ss = k.sumsq && k.rs_parts == nullptr ? 0.137 * nk : 0;
   int best = 256;
   *us = 1e30;
   for (const auto& c : shape) {
     const int64_t tiles = cdiv(k.M, c.bm) * k.tiles_n, rounds = cdiv(tiles, cus);
     const double fill = (double)tiles / (double)(rounds * cus);
-    const double t = (double)rounds * (nk * (c.c0 + c.c1 * fill) + c.e);
+    const double step = c.c0 + fill * (c.c1 + 0.107 * std::min(1.0, (double)rounds * nk / 256));
+    const double epi = ec.wide * (0.891 + 4.17 * fill) + 6.06 * ec.rope + 0.384 * (ec.outs - 1);
+    const double t = (double)rounds * (nk * step + c.e + epi) + own_ss;
     if (t < *us) {
       *us = t;
       best = c.bm;

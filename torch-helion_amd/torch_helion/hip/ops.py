@@ -185,6 +185,15 @@ def gemm(call: GemmCall, kernel: str | None = None) -> None:
     abi.check(lib.th_gemm(C.byref(d), _stream(call.lhs)), "th_gemm", kernel)
 
 
+def gemm_route(call: GemmCall) -> tuple[int, int, int, float]:
+    """(abi.LOOP_*, tile rows, packed tile columns) that th_gemm runs for this call, and the
+    time a bf16 loop is estimated to take (us on the device, 0.0 for the other types)."""
+    route, us = (C.c_int32 * 3)(), C.c_double()
+    d = call.descriptor()
+    abi.check(abi.load().th_gemm_route(C.byref(d), route, C.byref(us)), "th_gemm_route")
+    return route[0], route[1], route[2], us.value
+
+
 def gemm_noalloc(call: GemmCall, kernel: str | None = None) -> None:
     """th_gemm_noalloc: the same GEMM with the library's fixed per-GPU scratch in place of a
     workspace (``call.workspace`` is ignored); allocates nothing."""
