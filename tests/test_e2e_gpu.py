@@ -633,6 +633,7 @@ def test_llama_rotary_projections_merged(gpu, heads, kv_heads, seq, tmp_path):
         outs.append(res.run(*x)[0].clone())
         merged = [l for l in res.device_program.launches if "+" in l.kernel]
         assert len(merged) == (1 if merge is None else 0)
+        assert [(p.members, p.merged) for p in res.device_program.launch_merges] == [(l.info["merged"], True) for l in merged]
     torch.cuda.synchronize()
     # The products are the same sums in the same order. Two launches may run on another kernel than one, whose
     # fp32 row sums of squares add up in another order: the row scales then differ by a few 2^-24, which moves a
@@ -640,3 +641,23 @@ def test_llama_rotary_projections_merged(gpu, heads, kv_heads, seq, tmp_path):
     # at most: under 2^-8 of the result's 2-norm even if every value moved.
     a, b = outs[0].double(), outs[1].double()
     assert float((a - b).norm() / b.norm()) < 2.0**-8
+
+
+def test_llama_rotary_projections_priced(gpu, tmp_path):
+    """Where two launches of the rotary projections are estimated the faster (both fill whole rounds of tiles, one
+    does not), merge_siblings=None keeps them apart and says so in the plan; True merges all the same."""
+    from targets.llama_block import LlamaBlockConfig, build_llama_block
+    from torch_helion import CompileConfig, compile_model
+
+    cfg = LlamaBlockConfig(batch=4, seq=2048, hidden=2048, heads=32, kv_heads=8, intermediate=256, causal=True,
+                           dtype=torch.bfloat16)
+    model = build_llama_block(cfg, seed=3)
+    x = model.example_inputs(seed=3)
+    for merge in (None, True):
+        res = compile_model(model, x, CompileConfig(run_name=f"priced_{merge}", results_dir=tmp_path, device_check=False,
+                                                    reference_check=False, verify_passes=False, merge_siblings=merge))
+        merged = [l for l in res.device_program.launches if "+" in l.kernel]
+        price, = res.device_program.launch_merges
+        assert not price.merged and len(merged) == (1 if merge else 0)
+        plan = next(tmp_path.rglob(f"*priced_{merge}*/05_plan/plan.md"), None) or next(tmp_path.rglob("plan.md"))
+        assert " + ".join(price.members) in plan.read_text()

@@ -50,8 +50,9 @@ class CompileConfig:
     residual_fp32: bool = True                    # residual operands of GEMM epilogues travel in fp32
     merge_siblings: bool | None = None            # GEMM kernels sharing an lhs run as one launch (column windows);
                                                   # None: where the planner prices one launch below the separate
-                                                  # ones (optimizer/planner.py price_launch_merges; reported in
-                                                  # 05_plan/plan.md); True / False: always / never
+                                                  # ones (optimizer/planner.py price_launch_merges; bf16 rotary
+                                                  # projections: th_gemm's own estimates; reported in
+                                                  # 05_plan/plan.md) and e4m3 siblings; True / False: always / never
     cpu_flop_budget: float = 2e10                 # graphs above this skip CPU-side checks in "auto" mode
     reuse_buffers: bool = True                    # intermediates share device buffers by liveness
     merge_convs: bool = True                      # the depthwise convolutions feeding one SSD run as one launch

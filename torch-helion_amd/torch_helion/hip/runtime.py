@@ -188,7 +188,9 @@ class DeviceProgram:
             groups = {k: v for k, v in groups.items() if k in keep}
             away = {m[0].name for v in groups.values() for m in v[1:]}
         self._merge_groups, self._merged_away = groups, away
-        # (rotary siblings and e4m3 decode GEMMs: one launch always pays, see _plan_rotary_merges)
+        # rotary siblings and e4m3 decode GEMMs (_plan_rotary_merges); the bf16 ones priced
+        # when they are lowered, unless merge_siblings asks for every merge
+        self._price_rotary = merge_siblings is None
         self._rotary_groups = self._plan_rotary_merges(program, self._merged_away) if merge_siblings is not False else {}
         # scans whose only reader normalises them with a gain: the scan applies it (_plan_norm_folds)
         self._rs_parts: dict[tuple, torch.Tensor] = {}
@@ -215,7 +217,7 @@ class DeviceProgram:
             elif k.name in self._rotary_groups:
                 members = [m[0] for m in self._rotary_groups[k.name]]
                 merged = self._lower_rotary_merged(members)
-                if merged is None:  # the parts disagree: each member at the leader's position
+                if merged is None:  # the parts disagree, or two launches are faster: each member at the leader's position
                     merged = [x for m in members for x in self._lower(m)]
                 self.launches.extend(merged)
             else:
@@ -982,10 +984,11 @@ class DeviceProgram:
     # own column window (fused RoPE included: a head never straddles two windows).
     # e4m3 weights (decode programs): one activation-gain pre-pass and one reduce
     # pass instead of one per kernel. bf16 weights: q and k|v of a grouped-query
-    # block alone leave half the CUs idle at a few thousand rows (2000 rows, K =
-    # 2048: q 37 us on 128 .. 256 tiles, k|v 34 us on 64; together on 192 tiles
-    # 33 us) and fill the same rounds of tiles together that they fill apart at
-    # many rows.
+    # block alone leave CUs idle up to a few thousand rows (K = 2048, q 2048 and
+    # k|v 2 x 512 columns: 2000 rows 64.3 us in two launches, 37.8 in one; K = 4096,
+    # q 4096 and k|v 2 x 1024: 1000 rows 107 and 62.5, 16384 rows 698 and 666), but
+    # not at every size (K = 8192, q 8192 and k|v 2 x 1024, 4096 rows: 563 and 592):
+    # the sum of th_gemm's own estimates decides.
     def _plan_rotary_merges(self, program: Program, away: set[str]):
         produced_at = {o.tensor: i for i, k in enumerate(program.kernels) for o in k.outputs}
 
@@ -1085,6 +1088,23 @@ class DeviceProgram:
         if not fp8 and (rope is None or rope[3] < 64 or 256 % rope[3] or n_tot % 256 or n_tot < 2048):
             return None  # (256-column tiles of whole heads)
         names = [spec.name for spec, _ in parts]
+        if not fp8:
+            from ..optimizer.planner import LaunchMerge
+
+            def estimate(n, n_acc, outs, mask, pt) -> float:
+                call = ops.GemmCall(T, n, K, n_acc, p0["lhs"], p0["lhs"], outs, sumsq=p0["sumsq"], rscale_mask=mask)
+                if pt["rope"] is not None:
+                    call.rope_cos, call.rope_sin, call.rope_period, call.rope_head_dim = pt["rope"][:4]
+                return ops.gemm_route(call)[3]
+
+            # (two launches took about 5% longer, against the one, than the estimates say where both fill
+            # whole rounds of tiles: 16384 rows, K = 4096 698 and 666 us, estimated 707 and 709; the second
+            # one's ramp, and the lhs read again)
+            split_us = 1.05 * sum(estimate(pt["N"], pt["n_used"], pt["epi"], pt["mask"], pt) for _, pt in parts)
+            price = LaunchMerge(names, split_us, estimate(n_tot, 1, epi, 1 if p0["mask"] else 0, {"rope": rope}))
+            self.launch_merges.append(price)
+            if self._price_rotary and not price.merged:
+                return None
         info = {"n_acc": 1, "merged": names, "cols": n_tot, "ops": [x.op for x in epi], "rscale": p0["sumsq"],
                 "rope_fused": rope is not None}
         dt = _FP8 if fp8 else torch.bfloat16

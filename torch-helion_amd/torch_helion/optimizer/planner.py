@@ -235,7 +235,8 @@ def price_launch_merges(program: Program, groups: list[list[tuple[str, int]]], h
 def launch_merge_report(merges: list[LaunchMerge]) -> str:
     lines = ["## Launch merges (HIP backend)", "",
              "Sibling GEMM kernels reading one lhs, priced as separate launches and as one launch over",
-             "their concatenated weights (calibrated cost model, launch overhead included).", "",
+             "their concatenated weights (calibrated cost model, launch overhead included; bf16 rotary",
+             "projections by th_gemm's own estimates).", "",
              "| kernels | split us | merged us | decision |", "|---|---:|---:|---|"]
     for m in merges:
         lines.append(f"| {' + '.join(m.members)} | {m.split_us:,.1f} | {m.merged_us:,.1f} | "
