@@ -113,3 +113,11 @@ def test_estimate_counts_the_steps_that_run():
 @pytest.mark.parametrize("N,K,form", [(8192, 256, "swiglu"), (2048, 192, "acc"), (1024, 2048, "add_fp32"), (4096, 4096, "add")])
 def test_a_copy_beside_an_output_changes_nothing(M, N, K, form):
     assert ops.gemm_route(_call(M, N, K, form)) == ops.gemm_route(_call(M, N, K, form, copy32=True))
+
+
+@pytest.mark.parametrize("M,N,K,slices", [(32, 64, 256, 8), (32, 64, 260, 9), (128, 512, 512, 16), (32, 64, 16384, 64)])
+def test_fp32_workspace_holds_the_slices_that_run(M, N, K, slices):
+    """fp32 split-K: slices are whole 32-wide steps, so no more of them are asked for than K has steps."""
+    bn = 64 if N <= 64 else 128
+    Mp, Npk = -(-M // 32) * 32, -(-N // bn) * bn
+    assert ops.gemm_workspace_bytes(M, N, K, 1, torch.float32) == slices * Mp * (Npk + 1) * 4

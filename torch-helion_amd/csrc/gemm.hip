@@ -1457,13 +1457,13 @@ __global__ void __launch_bounds__(256) gemm_f32_ksr_kernel(F32Ksp q) {
 }
 
 // K slices of the split-K fp32 path for tiles 32-row x BNC tiles: about one
-// workgroup per CU, each slice at least half a 32-wide step. (Two per CU measured
+// workgroup per CU, each slice whole 32-wide steps (the last one the rest). (Two per CU measured
 // 15% slower on the fp32 block: twice the partial sums to write and re-read,
 // each workgroup's K slice little more than its load pipeline's depth.)
 static int f32_ksp_slices(int64_t tiles, int64_t K) {
   const int64_t cus = device_cus() > 0 ? device_cus() : 256;
   const int64_t want = cdiv(cus, tiles);
-  return (int)std::max((int64_t)1, std::min({want, cdiv(K, 16), (int64_t)64}));
+  return (int)std::max((int64_t)1, std::min({want, cdiv(K, 32), (int64_t)64}));
 }
 
 static int64_t f32_ksp_bytes(int64_t M, int64_t Npk, int64_t K, int bnc) {

@@ -153,14 +153,14 @@ def _gemm_compose(hw: HardwareSpec, T: int, N: int, K: int, n_acc: int, dtype: s
                   detail: dict[str, Any]) -> CostBreakdown:
     """bf16 / fp32 GEMM of T x (n_acc N) x K on the HIP kernel's tiles."""
     flops = 2.0 * T * N * K * n_acc
-    bm, bn = gemm_tiles(N, n_acc, T, dtype, hw.compute_units)
+    bm, bn = gemm_tiles(N, n_acc, T, dtype, hw.compute_units, K)
     tiles_m, tiles_n = math.ceil(T / bm), math.ceil(N / bn)
     kq = math.ceil(K / (16 if dtype == "float32" else 64)) * (16 if dtype == "float32" else 64)
     if dtype == "float32" and tiles_m * tiles_n < hw.compute_units:
         # fp32 grids too small for the GPU: 32-row tiles, K split over about one
         # workgroup per CU (th_gemm's workspace path), a second pass sums the slices
         tiles_m = math.ceil(T / 32)
-        ksg = max(1, min(math.ceil(hw.compute_units / (tiles_m * tiles_n)), math.ceil(K / 16), 64))
+        ksg = max(1, min(math.ceil(hw.compute_units / (tiles_m * tiles_n)), math.ceil(K / 32), 64))
         mfma = 2.0 * tiles_m * 32 * tiles_n * bn * n_acc * kq
         return _compose(hw, flops, nbytes, mfma, tiles_m * tiles_n * ksg, dtype,
                         {"tile_t": 32, "tile_n": bn, "k_slices": ksg}, detail, "gemm_fp32",
