@@ -72,14 +72,6 @@ __device__ __forceinline__ void lds_barrier() {
   barrier_keep_loads();
 }
 
-// The lane id, computed anew where it is asked for: what is derived from it there
-// is not kept in registers across a loop that has none to spare.
-__device__ __forceinline__ int fresh_lane() {
-  int l;
-  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
-  return l;
-}
-
 // ------------------------------------------------------------ bf16 helpers
 __device__ __forceinline__ float bf16_to_f32(uint16_t h) {
   return __uint_as_float(((uint32_t)h) << 16);

@@ -443,7 +443,7 @@ __global__ void __launch_bounds__(512) gemm_fp8_lds_kernel(Fp8K p) {
   constexpr int SLB = ROWS * RB;       // bytes per activation slice
   constexpr int NWV = 8;               // waves per workgroup: 4 column groups x 2 K halves
   constexpr int NT = 64 * NWV;         // threads per workgroup
-  constexpr int P = 2;                 // slices in flight ahead of the MFMAs (measured best of 2, 3, 5)
+  constexpr int P = 2;                 // slices in flight ahead of the MFMAs (best of 2, 3 and 5 in a four-wave kernel; not swept in this one)
   constexpr int NBUF = P + 1;          // slice buffers (LDS) and weight register slots
   constexpr int ALD = SLB / 1024 / NWV;  // activation loads per wave per slice
   constexpr int RPI = 1024 / RB;       // rows per activation load

@@ -138,44 +138,8 @@ __device__ __forceinline__ void store4(void* p, int64_t off, int dtype, bool vec
   for (int q = 0; q < 4 && q < valid; ++q) store_elem(p, off + q, dtype, t[q]);
 }
 
-// Block id -> output tile. Consecutive workgroups are dealt round-robin to the
-// 8 XCDs; remap so each XCD owns a contiguous range of logical tiles, then walk
-// that range in groups of 8 tile-rows so neighbouring blocks on one XCD share
-// lhs rows and rhs columns in that XCD's L2.
-__device__ __forceinline__ void map_tile_id(int pid, int tiles_m, int tiles_n, int& tm, int& tn) {
-  const int nb = tiles_m * tiles_n;
-  if ((nb & 7) == 0) pid = (pid & 7) * (nb >> 3) + (pid >> 3);
-  const int G = 8;
-  const int group = pid / (G * tiles_n);
-  const int first = group * G;
-  const int gm = min(tiles_m - first, G);
-  const int in_group = pid - group * G * tiles_n;
-  tm = first + in_group % gm;
-  tn = in_group / gm;
-}
-
 // 8 consecutive elements (one 16-byte bf16 or two 16-byte fp32 accesses when
 // vec8, element by element for a ragged end or unaligned rows).
-__device__ __forceinline__ void load8(const void* p, int64_t off, int dtype, bool vec8, int valid, float* v) {
-  if (vec8 && valid >= 8) {
-    if (dtype == TH_BF16) {
-      const uint4 w = *(const uint4*)((const uint16_t*)p + off);
-      const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        v[2 * q] = __uint_as_float(ws[q] << 16);
-        v[2 * q + 1] = __uint_as_float(ws[q] & 0xffff0000u);
-      }
-    } else {
-      const float4 a = *(const float4*)((const float*)p + off), b = *(const float4*)((const float*)p + off + 4);
-      v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-    }
-    return;
-  }
-#pragma unroll
-  for (int q = 0; q < 8; ++q) v[q] = q < valid ? load_elem(p, off + q, dtype) : 0.f;
-}
-
 __device__ __forceinline__ void store8(void* p, int64_t off, int dtype, bool vec8, int valid, const float* v) {
   if (vec8 && valid >= 8) {
     if (dtype == TH_BF16) {
@@ -200,16 +164,6 @@ __device__ __forceinline__ void store8(void* p, int64_t off, int dtype, bool vec
 // window; only the destination differs).
 __host__ __device__ __forceinline__ bool same_values(const EpiOutK& x, const EpiOutK& y) {
   return x.op == y.op && x.a == y.a && x.b == y.b && x.e == y.e && x.cb == y.cb && x.ce == y.ce;
-}
-
-// Sum of squares of an MFMA operand fragment (8 bf16) with v_dot2_f32_bf16:
-// each bf16 product is exact in fp32, accumulation is fp32.
-__device__ __forceinline__ float sumsq8_dot(bf16x8_t v, float acc) {
-  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_shufflevector(v, v, 0, 1), __builtin_shufflevector(v, v, 0, 1), acc, false);
-  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_shufflevector(v, v, 2, 3), __builtin_shufflevector(v, v, 2, 3), acc, false);
-  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_shufflevector(v, v, 4, 5), __builtin_shufflevector(v, v, 4, 5), acc, false);
-  acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_shufflevector(v, v, 6, 7), __builtin_shufflevector(v, v, 6, 7), acc, false);
-  return acc;
 }
 
 // What a GEMM's epilogue adds to the time of a tile, in the terms of the estimates that

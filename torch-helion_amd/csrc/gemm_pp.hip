@@ -67,6 +67,14 @@ __device__ __forceinline__ void pp_map(int L, int tiles_m, int tiles_n, int& tm,
   tn = in_group / gm;
 }
 
+// The lane id, computed anew where it is asked for: what is derived from it there
+// is not kept in registers across a loop that has none to spare.
+__device__ __forceinline__ int fresh_lane() {
+  int l;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+  return l;
+}
+
 // The kernel's arguments, read anew where they are asked for: values derived from
 // them (and from the lane id, fresh_lane) per tile would otherwise be kept in
 // registers across the K loop, which has none to spare (spilled, their reload in
