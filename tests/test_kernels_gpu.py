@@ -63,7 +63,8 @@ def test_gemm_bf16_plain(gpu, M, N, K):
 
 @pytest.mark.parametrize("M,N,K,n_acc", [(8200, 4096, 1024, 1), (2000, 768, 4096, 2), (777, 1024, 2048, 4)])
 def test_gemm_bf16_deep_k_ragged_m(gpu, M, N, K, n_acc):
-    """Many 64-wide K tiles, M not a multiple of the row tile (256-row tiles at 8200 x 4096), RMS fold on."""
+    """Many 64-wide K tiles, M not a multiple of the row tile (192-row ping-pong tiles at 8200 x 4096, 128-row ones
+    at 2000 x 2 * 768, the 64-row direct loop with four accumulators), RMS fold on."""
     from torch_helion.hip import abi, ops
 
     announce(f"gemm bf16 deep-K M={M} N={N} K={K} n_acc={n_acc}")
@@ -140,10 +141,11 @@ def test_gemm_bf16_large_tiles(gpu, M, N, K, n_acc):
 @pytest.mark.parametrize("M,N,K,n_acc,mask", [(2000, 2192, 512, 1, 1), (2048, 2192, 512, 1, 0), (1000, 5000, 256, 1, 1),
                                               (2040, 1100, 512, 2, 2), (2048, 1100, 512, 1, 1), (2000, 700, 512, 1, 1)])
 def test_gemm_direct_two_blocks_per_cu(gpu, M, N, K, n_acc, mask):
-    """64-row tiles numbering between one and two per CU (288, 288, 320, 288, 288 and 352 tiles of
-    64 x 256, 64 x 256, 64 x 256, 64 x 2 x 128, 64 x 128 and 64 x 64) run the direct loop with
-    stages within 80 KiB, two workgroups per CU, the row scales kept in the stage memory:
-    RMS-scaled and plain accumulators, the sums of squares, a ragged M and N."""
+    """64-row tiles numbering between one and two per CU (the last three cases: 288, 288 and 352 tiles of
+    64 x 2 x 128, 64 x 128 and 64 x 64) run the direct loop with stages within 80 KiB, two workgroups per
+    CU, the row scales kept in the stage memory: RMS-scaled and plain accumulators, the sums of squares, a
+    ragged M and N. The first three run on 128-row ping-pong tiles (one accumulator on 64 x 256 direct
+    tiles: test_gemm_older_loops_gpu.py)."""
     from torch_helion.hip import abi, ops
 
     announce(f"gemm bf16 direct two per CU M={M} N={N} K={K} n_acc={n_acc} mask={mask}")
@@ -300,7 +302,8 @@ def test_gemm_rope_whole_heads_per_wave(gpu, hd, n_acc):
 def test_gemm_kv_rope_head_wider_than_half_tile(gpu, S):
     """k and v projections in one launch (two accumulators, 128-column tiles) with RoPE on k at head_dim 128:
     a head spans both column halves of the tile, so each wave holds one whole accumulator instead. M = 8 S
-    rows selects 128-row (S=512) and 256-row (S=2048) persistent tiles. RMS fold on both accumulators."""
+    rows selects 128-row ping-pong tiles (S=512) and 256-row persistent ones (S=2048). RMS fold on both
+    accumulators."""
     from torch_helion.hip import abi, ops
 
     B, Hkv, hd, K, eps = 8, 8, 128, 512, 1e-5
@@ -628,10 +631,9 @@ def test_gemm_extra_ops(gpu):
 
 @pytest.mark.parametrize("M", [16384, 16300])
 def test_gemm_whole_wave_wide_tiles(gpu, M):
-    """One accumulator over 1024 columns at 64 row tiles of 256: exactly one wave of
-    256 x 256 tiles on a 256-CU device, the tile th_gemm then takes instead of two
-    256 x 128 tiles per CU (the Mamba-2 out-projection with its fp32 residual; a ragged
-    last row tile in the second case)."""
+    """One accumulator over 1024 columns (packed for 128-column tiles) at 64 row tiles of 256: exactly one
+    wave of 256 x 256 ping-pong tiles on a 256-CU device (the Mamba-2 out-projection with its fp32
+    residual; a ragged last row tile in the second case)."""
     from torch_helion.hip import abi, ops
 
     announce(f"gemm bf16 whole-wave 256x256 tiles M={M}")
@@ -973,7 +975,7 @@ def test_ssd_output_gain_and_row_sums(gpu, bs, s, h, p, n, g, chunk):
     assert _rel(parts, ref) < 1e-6
 
 
-@pytest.mark.parametrize("M,N,K", [(16384, 1024, 2048), (300, 512, 256)])  # persistent 256 x 256; direct loop
+@pytest.mark.parametrize("M,N,K", [(16384, 1024, 2048), (300, 512, 256)])  # ping-pong 256 x 256; direct loop
 def test_gemm_row_sums_from_producer(gpu, M, N, K):
     """rs_parts: the row scale from the lhs producer's partial sums of squares (of the values
     before its gain) instead of the GEMM's own sum over its lhs. With parts that are the
