@@ -8,21 +8,31 @@ from __future__ import annotations
 import dataclasses
 
 import pytest
+import torch
 
 
 def test_gemm_tiles_mirror_th_gemm():
-    """th_gemm's rules (csrc/gemm.hip): 256-row tiles when they give two blocks per CU,
-    128 when one, else 64; one accumulator over a multiple of 256 columns takes
-    256 x 256 tiles when those make whole waves of the 256 CUs."""
+    """The tile that th_gemm says it would run (th_gemm_route; no GPU), over rows, columns and depths on both
+    sides of every rule: 64-, 128- and 256-row loops, ping-pong rows, partial K steps, ragged columns."""
+    from test_gemm_route import _Fake
     from torch_helion.cost_models.roofline import gemm_tiles
+    from torch_helion.hip import abi, ops
 
-    assert gemm_tiles(1024, 1, 16384, "bfloat16") == (256, 256)   # 64 x 4 = 256 tiles: one whole wave
-    assert gemm_tiles(1280, 1, 16384, "bfloat16") == (256, 128)   # 64 x 5 = 320: not whole waves
-    assert gemm_tiles(1024, 1, 8192, "bfloat16") == (128, 128)    # 128 wide tiles: too few
-    assert gemm_tiles(1000, 1, 16384, "bfloat16") == (256, 128)   # not a multiple of 256 columns
-    assert gemm_tiles(2048, 2, 16384, "bfloat16") == (256, 128)   # two accumulators: unchanged
-    assert gemm_tiles(4096, 1, 16384, "bfloat16") == (256, 256)
-    assert gemm_tiles(512, 1, 64, "bfloat16") == (64, 64)
+    if not abi.library_path().exists():
+        pytest.skip("libth_hip.so not built (run __graft_entry__.build())")
+    bf = torch.bfloat16
+    seen = set()
+    for n_acc in (1, 2, 3):
+        for N in (48, 512, 768, 1000, 1024, 1280, 2048, 4096, 8200, 50280):
+            for K in (64, 192, 576, 1000, 2048, 14336):
+                for M in (1, 64, 300, 1500, 4096, 8192, 16384):
+                    outs = [ops.EpiSpec(abi.EPI_ACC, _Fake(M, N, bf), a=i) for i in (0,)]
+                    loop, bm, cols, _ = ops.gemm_route(ops.GemmCall(M, N, K, n_acc, _Fake(M, K, bf), _Fake(N, K, bf), outs))
+                    assert gemm_tiles(N, n_acc, M, "bfloat16", 256, K) == (bm, cols // n_acc), (M, N, K, n_acc)
+                    seen.add((loop, bm))
+    assert {l for l, _ in seen} == {abi.LOOP_BF16_STAGED, abi.LOOP_BF16_DIRECT, abi.LOOP_BF16_PERSISTENT,
+                                    abi.LOOP_BF16_PINGPONG}
+    assert {bm for l, bm in seen if l == abi.LOOP_BF16_PINGPONG} == {128, 192, 256}
 
 
 def _rec(kernel, cat, ideal, waves, measured):
@@ -50,6 +60,18 @@ def test_calibration_fit_recovers_parameters():
     assert c["kernels_fitted"] == {"gemm_bf16": 7, "gemm_bf16_merged": 3}
     for r in recs:
         assert predict(r, c) == pytest.approx(r["measured_us"], rel=2e-3)
+
+
+def test_calibration_counts_a_repeated_shape_once():
+    """24 equal layers whose shape does not follow the other kernels' line move the fit no further than one."""
+    from torch_helion.cost_models.calibrate import distinct, fit
+
+    recs = [_rec(f"k{i}", "gemm_bf16", ideal, waves, 2 * ideal + 10 * waves + 8)
+            for i, (ideal, waves) in enumerate([(5, 1), (40, 2), (100, 4), (300, 4), (800, 8), (20, 0.25)])]
+    odd = [_rec(f"layer{i}", "gemm_bf16", 27.0, 1.0, 90.0 + i) for i in range(25)]
+    d = distinct(recs + odd)
+    assert len(d) == 7 and d[-1]["measured_us"] == 102.0
+    assert fit(d) == fit(recs + [{**odd[0], "measured_us": 102.0}])
 
 
 def test_calibration_without_merged_samples_has_no_factor():

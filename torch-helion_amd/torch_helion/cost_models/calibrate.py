@@ -15,7 +15,7 @@ output tiles, scaled by the tile's area against 256 x 256 (pipeline fill and
 epilogue: what makes a K = 1024 GEMM slower per FLOP than a K = 4096 one, and
 a 64-row tile cheaper per wave than a 256-row one). ``fit`` takes runs that carry both the program
 (``06_opir.json``) and measured per-kernel times (``11_bench.json``, written by
-the bench stage or bench.py) and returns
+the bench stage or bench.py), each distinct shape of a run once, and returns
 
 * ``launch_overhead_us``: the median time of kernels whose ideal time is
   under 1 µs (their time is launch and latency, not work), the fixed part of
@@ -82,7 +82,16 @@ def samples(run_dirs: list[Path], hw: HardwareSpec) -> list[dict[str, Any]]:
                         "ideal_us": max(c.t_mfma_us, c.t_hbm_us),
                         "waves": c.waves * c.detail.get("wave_scale", 1.0), "measured_us": float(m["us"]),
                         "bound": c.bound})
-    return out
+    return distinct(out)
+
+
+def distinct(recs: list[dict[str, Any]]) -> list[dict[str, Any]]:
+    """One record per shape of a run, at its median time: the 24 equal layers of a backbone
+    would otherwise outweigh every other kernel of the fit 24 to one."""
+    groups: dict[tuple, list[dict[str, Any]]] = {}
+    for r in recs:
+        groups.setdefault((r["run"], r["category"], round(r["ideal_us"], 3), round(r["waves"], 4)), []).append(r)
+    return [{**g[0], "measured_us": statistics.median(r["measured_us"] for r in g)} for g in groups.values()]
 
 
 def _merged_sample(name: str, m: dict[str, Any], specs: dict[str, Any], prog: Program,

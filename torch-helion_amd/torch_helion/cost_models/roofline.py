@@ -65,24 +65,54 @@ def _bytes(t: TensorType) -> int:
     return t.numel * DTYPE_BYTES.get(t.dtype, 4)
 
 
-def gemm_tiles(N: int, n_acc: int, M: int, dtype: str, cus: int = 256) -> tuple[int, int]:
-    """(BM, per-accumulator column tile) the HIP GEMM picks (mirrors th_gemm in csrc/gemm.hip:
-    256-row tiles when they still give two blocks per CU, 128 when they give one, else 64;
-    one accumulator over a multiple of 256 columns takes 256 x 256 tiles when they make
-    whole waves)."""
+def gemm_tiles(N: int, n_acc: int, M: int, dtype: str, cus: int = 256, K: int = 4096) -> tuple[int, int]:
+    """(BM, per-accumulator column tile) that the HIP GEMM picks for plain outputs (mirrors
+    th_gemm in csrc/gemm.hip and gemm_pp_rows in csrc/gemm_pp.hip, estimates and constants
+    included; ``th_gemm_route`` is the original)."""
     if dtype == "float32":
         bn = {1: 128 if N > 64 else 64, 2: 64 if N > 32 else 32, 3: 64}.get(n_acc, 64 if N > 32 else 32)
         return 64, bn
     bn = {1: 256 if N >= 2048 else (128 if N >= 768 else 64), 2: 128 if N >= 128 else (64 if N > 32 else 32),
           3: 64}.get(n_acc, 64 if N > 32 else 32)
-    if n_acc == 1 and bn == 128 and N % 256 == 0:
-        t256 = math.ceil(M / 256) * (N // 256)
-        if t256 >= cus and t256 % cus == 0:    # whole waves of 256 x 256 tiles
-            return 256, 256
     tn = math.ceil(N / bn)
-    if math.ceil(M / 256) * tn >= 2 * cus:
-        return 256, bn
-    return (128 if math.ceil(M / 128) * tn >= cus else 64), bn
+    bm = 256 if math.ceil(M / 256) * tn >= 2 * cus else 128 if math.ceil(M / 128) * tn >= cus else 64
+    wide = n_acc == 1 and bn == 128 and N % 256 == 0    # one accumulator's packed columns are in order
+    if K >= 128 and N % 8 == 0 and n_acc <= 2 and (bn * n_acc == 256 or wide):
+        rows, us = _pingpong_rows(M, N // 256 if wide else tn, K, cus)
+        if K % 64 or us < _loop_us(M, N, tn, K, bm, bn * n_acc, cus):
+            return rows, 256 // n_acc
+    return (128 if bm == 64 and K % 64 else bm), bn
+
+
+def _rounds(M: int, tn: int, bm: int, cus: int) -> tuple[int, float]:
+    tiles = math.ceil(M / bm) * tn
+    rounds = math.ceil(tiles / cus)
+    return rounds, tiles / (rounds * cus)
+
+
+def _pingpong_rows(M: int, tn: int, K: int, cus: int) -> tuple[int, float]:
+    nk = 2 * math.ceil(K / 128)
+    best = (256, math.inf)
+    for bm, c0, c1, e in ((256, 0.868, 0.570, 12.0), (192, 0.611, 0.454, 9.91), (128, 0.465, 0.243, 8.14)):
+        rounds, fill = _rounds(M, tn, bm, cus)
+        us = rounds * (nk * (c0 + fill * (c1 + 0.107 * min(1.0, rounds * nk / 256))) + e)
+        best = min(best, (bm, us), key=lambda x: x[1])
+    return best
+
+
+def _loop_us(M: int, N: int, tn: int, K: int, bm: int, cols: int, cus: int) -> float:
+    nk, full = math.ceil(K / 64), cols > 128
+    rounds, fill = _rounds(M, tn, bm, cus)
+    if bm == 64:
+        tiles = math.ceil(M / 64) * tn
+        load = tiles / cus
+        if tiles > cus:
+            return 4.784 + 1.3 * load + math.ceil(tiles / (2 * cus)) * nk * (1.13 if full else 0.557)
+        return 4.4 + 1.3 * load + nk * (0.756 + 0.512 * max(0.0, load - 0.7) if full else 0.419)
+    busy = fill * min(1.0, rounds * nk / 256)
+    if bm == 256:
+        return rounds * (nk * (1.12 + 0.413 * fill + 0.172 * busy) + 10.5 + (1.53 * fill if N % 64 else 0.0))
+    return rounds * ((nk * (0.692 + 0.261 * fill) + 8.14 if full else max(7.59, 0.892 * nk)) + 0.0247 * nk * busy)
 
 
 def category(spec: KernelSpec, tensors: dict[str, TensorType]) -> str:
