@@ -23,7 +23,7 @@ def test_gemm_tiles_mirror_th_gemm():
     bf = torch.bfloat16
     seen = set()
     for n_acc in (1, 2, 3):
-        for N in (48, 512, 768, 1000, 1024, 1280, 2048, 4096, 8200, 50280):
+        for N in (48, 128, 512, 768, 1000, 1024, 1280, 2048, 4096, 8200, 50280):
             for K in (64, 192, 576, 1000, 2048, 14336):
                 for M in (1, 64, 300, 1500, 4096, 8192, 16384):
                     outs = [ops.EpiSpec(abi.EPI_ACC, _Fake(M, N, bf), a=i) for i in (0,)]

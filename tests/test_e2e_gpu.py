@@ -641,6 +641,10 @@ def test_llama_rotary_projections_merged(gpu, heads, kv_heads, seq, tmp_path):
     # at most: under 2^-8 of the result's 2-norm even if every value moved.
     a, b = outs[0].double(), outs[1].double()
     assert float((a - b).norm() / b.norm()) < 2.0**-8
+    # And row by row, so that no few rows are wrong: the output's own rounding (2^-8 of the row), and four bf16
+    # roundings in a row in what is added to the residual (projections, attention output, MLP input and operand).
+    d, r = a - b, b - x[0].to(b.device).double().reshape(b.shape)
+    assert bool((d.norm(dim=-1) < 2.0**-8 * b.norm(dim=-1) + 4 * 2.0**-8 * r.norm(dim=-1)).all())
 
 
 def test_llama_rotary_projections_priced(gpu, tmp_path):

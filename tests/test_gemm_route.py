@@ -28,7 +28,9 @@ class _Fake:
 def _call(M, N, K, form, copy32=False):
     bf, f32, E = torch.bfloat16, torch.float32, ops.EpiSpec
     n_acc, kw, w = 1, {}, []
-    if form == "acc":
+    if form == "acc2":
+        n_acc, outs = 2, [E(abi.EPI_ACC, _Fake(M, N, bf)), E(abi.EPI_ACC, _Fake(M, N, bf), a=1)]
+    elif form == "acc":
         outs = [E(abi.EPI_ACC, _Fake(M, N, bf))]
     elif form in ("add", "add_fp32", "add_parts"):
         outs = [E(abi.EPI_ADD, _Fake(M, N, bf), e=0)]
@@ -78,6 +80,7 @@ D, P, PP = abi.LOOP_BF16_DIRECT, abi.LOOP_BF16_PERSISTENT, abi.LOOP_BF16_PINGPON
     (16384, 2048, 192, "acc", (P,)),            # - / 29.5 / 33.5
     (16384, 2048, 320, "acc", (P,)),            # - / 36.1 / 41.5
     (16384, 2048, 576, "acc", (P,)),            # - / 48.5 / 51.9
+    (16384, 128, 1024, "acc2", (D,)),           # 25.0 / - / 27.1 (after the kernel that writes the lhs)
     (2067, 20352, 256, "add", (PP,)),           # - / 74.1 / 53.7
     (16384, 2192, 512, "windows", (PP,)),       # - / 86.2 / 68.0
     (500, 2192, 512, "windows", (PP,)),         # 16.8 / - / 15.4

@@ -2084,6 +2084,10 @@ static int gemm_run(const th_gemm_desc* d, void* stream, int32_t* route, double*
     if (gemm_pp_fits(kp)) {
       double t_pp = 0;
       const int pbm = gemm_pp_rows(kp, ec, cus, &t_pp);
+      // One column tile: the lhs is read once, in a model from beyond the L2s, and twice the
+      // workgroups on 64 rows fetch it sooner (Mamba's B | C, 16384 x 2 * 128 x 1024: 25.0 us after
+      // the kernel that wrote the lhs, 27.1 on 128-row tiles; with the lhs at hand 17.4 and 15.9).
+      if (bm == 64 && kp.tiles_n == 1) t_pp = std::max(t_pp, 8.5 + (double)(pbm * d->K * 2) / 14e3);
       if (!direct || (bm > 64 && !wave_epi) || t_pp < t_loop) {
         if (us != nullptr) *us = t_pp;
         if (only_route(TH_LOOP_BF16_PINGPONG, pbm, 256)) return TH_OK;

@@ -79,6 +79,8 @@ def gemm_tiles(N: int, n_acc: int, M: int, dtype: str, cus: int = 256, K: int = 
     wide = n_acc == 1 and bn == 128 and N % 256 == 0    # one accumulator's packed columns are in order
     if K >= 128 and N % 8 == 0 and n_acc <= 2 and (bn * n_acc == 256 or wide):
         rows, us = _pingpong_rows(M, N // 256 if wide else tn, K, cus)
+        if bm == 64 and not wide and tn == 1:           # the lhs is read once, from beyond the L2s
+            us = max(us, 8.5 + rows * K * 2 / 14e3)
         if K % 64 or us < _loop_us(M, N, tn, K, bm, bn * n_acc, cus):
             return rows, 256 // n_acc
     return (128 if bm == 64 and K % 64 else bm), bn
