@@ -1088,7 +1088,7 @@ class DeviceProgram:
         if not fp8 and (rope is None or rope[3] < 64 or 256 % rope[3] or n_tot % 256 or n_tot < 2048):
             return None  # (256-column tiles of whole heads)
         names = [spec.name for spec, _ in parts]
-        if not fp8:
+        if not fp8 and self._price_rotary:
             from ..optimizer.planner import LaunchMerge
 
             def estimate(n, n_acc, outs, mask, pt) -> float:
@@ -1103,7 +1103,7 @@ class DeviceProgram:
             split_us = 1.05 * sum(estimate(pt["N"], pt["n_used"], pt["epi"], pt["mask"], pt) for _, pt in parts)
             price = LaunchMerge(names, split_us, estimate(n_tot, 1, epi, 1 if p0["mask"] else 0, {"rope": rope}))
             self.launch_merges.append(price)
-            if self._price_rotary and not price.merged:
+            if not price.merged:
                 return None
         info = {"n_acc": 1, "merged": names, "cols": n_tot, "ops": [x.op for x in epi], "rscale": p0["sumsq"],
                 "rope_fused": rope is not None}
